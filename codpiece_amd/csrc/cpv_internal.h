@@ -306,7 +306,7 @@ cpv_status cpv_qgemm_act(cpv_ctx* ctx, const cpv_weight* w, const cpv_act* act, 
 // act->m rows in one launch; cpv_qgemm_act takes them above 16 rows for
 // Q4_K and above 8 for Q6_K and Q8_0 (cpv_qgemm_wide_ok).
 bool cpv_qgemm_wide_ok(const cpv_weight* w, int64_t m);
-cpv_status cpv_qgemm_wide(cpv_ctx* ctx, const cpv_weight* w, const cpv_act* act, double* gsum, int win);
+cpv_status cpv_qgemm_wide(cpv_ctx* ctx, const cpv_weight* w, const cpv_act* act, double* gsum, int win, float* y);
 
 // A GEMM result kept in the accumulator for a fused consumer: row m, output n
 // is cpv_gout_value(acc[m * n_pad + n], ew[n], Ea(m), win) with Ea(m) the

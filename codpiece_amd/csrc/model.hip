@@ -539,7 +539,7 @@ __global__ __launch_bounds__(RB) void row_kernel(RowArgs a)
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
                     const int vq = (int)rintf(iscale * x[k]);
-                    q[k] = vq < 127 ? vq : 127;
+                    q[k] = (int8_t)(vq < 127 ? vq : 127);   // (the code as stored: what the sums add)
                 }
                 d = 1.0f / iscale;
             } else {
@@ -691,7 +691,7 @@ __global__ __launch_bounds__(256) void unit_kernel(RowArgs a)
         if (ax > 0.0f) {
             const float iscale = -127.0f / sx;
             const int vq = (int)rintf(iscale * val);
-            q = vq < 127 ? vq : 127;
+            q = (int8_t)(vq < 127 ? vq : 127);   // (the code as stored: what the sums add)
             d = 1.0f / iscale;
         }
         qa[(int64_t)m * Kp + e] = (int8_t)q;

@@ -73,7 +73,7 @@ __global__ __launch_bounds__(256) void quant_q8k_kernel(const float* __restrict_
     if (amax > 0.0f) {
         const float iscale = -127.0f / sx[imax];
         const int vq = (int)rintf(iscale * v);
-        q = vq < 127 ? vq : 127;
+        q = (int8_t)(vq < 127 ? vq : 127);   // (the code as stored: what the sums below add)
         d = 1.0f / iscale;
     }
     const int64_t Kp = (int64_t)U * 256;
@@ -1107,10 +1107,11 @@ static cpv_status qgemm_into(cpv_ctx* ctx, const cpv_weight* w, const cpv_act* a
                                      : lds_of<CPV_Q8_0>(M, a.nu_max, a.nt_max);
     };
     if (cpv_qgemm_wide_ok(w, m)) {
-        if ((st = cpv_qgemm_wide(ctx, w, act, a.gsum, a.win)) != CPV_OK) return st;
-        if (y)
+        const bool own = w->type != CPV_Q8_0;   // (the K-quants' kernel writes y itself)
+        if ((st = cpv_qgemm_wide(ctx, w, act, a.gsum, a.win, own ? y : nullptr)) != CPV_OK) return st;
+        if (y && !own)
             qgemm_finalize_kernel<<<dim3((unsigned)((w->n + 255) / 256), (unsigned)m), 256, 0, ctx->stream>>>(
-                a.gsum, a.n_pad, a.ew, a.da, kq ? U : 8 * U, 0, a.win, y, w->n);
+                a.gsum, a.n_pad, a.ew, a.da, 8 * U, 0, a.win, y, w->n);
         CPV_HIP(ctx, hipGetLastError());
         return CPV_OK;
     }

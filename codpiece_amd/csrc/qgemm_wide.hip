@@ -1,29 +1,24 @@
-// qgemm_wide.hip — the GEMMs for many activation rows (prompt prefill): Q4_K
-// first, then Q8_0 and Q6_K (below) on the same mapping.
+// qgemm_wide.hip — the GEMMs for many activation rows (prompt prefill, wide
+// verifies): Q4_K and Q6_K on one kernel, Q8_0 on its own.
 //
 // The prefill pushes a chunk of the prompt through the trunk as one batch of
 // rows (engine.rs:1922-1953, step_greedy -> run_general, qwen35.rs:1125-1302),
 // so every ggml_mul_mat there has tens to hundreds of activation rows.  The
 // numbers are exactly those of the skinny kernel (qgemm.hip): for activation
-// row m, weight row n and 256-element unit u,
+// row m, weight row n and 256-element unit u (Q4_K)
 //     isum = sum_j sc_j * dot_j      imin = sum_j mn_j * (codes of sub-block j)
 //     term = rint(dws * da * isum) - rint(dms * da * imin)        (binary64)
-// and the terms of all units are summed exactly into the same accumulator
-// entry, so the finalize kernel and the fused consumers of a kept result are
-// shared and the outputs are bit-identical to the skinny path's.
+// and the terms of all units are summed exactly, so the outputs are
+// bit-identical to the skinny path's whatever the split.
 //
-// Mapping.  A workgroup of 4 waves owns one 64-row weight tile and 64
-// activation rows (and, when the grid would be small, one slice of K).  Wave w
-// takes weight rows 16w..16w+15 against all 64 activation rows: four 16 x 16
-// output blocks.  Per unit and 32-element sub-block j it runs two 16x16x32
-// int8 MFMAs per block, one against the sub-block's 4-bit codes (the dots,
-// scaled by sc_j on the VALU) and one against mn_j in every byte, which sums
-// to imin directly (sum over k of a_k * mn_j(k)).  The activation codes of one
-// unit are staged in LDS for all four waves, double-buffered, while the next
-// unit's codes and weights are in flight.  The lane layout of the MFMA (A row
-// and B column = lane % 16, 8 consecutive k per lane >> 4, C rows 4 (lane >>
-// 4) + i of column lane % 16) puts one weight row in each lane, so its scales
-// are decoded once per unit.
+// Mapping.  A workgroup of 4 waves owns one 64-row weight tile and up to 128
+// activation rows (Q8_0: 64), over all of K or one slice of it.  Wave w takes
+// weight rows 16w..16w+15 against all of them, in 16 x 16 output blocks.  The
+// activation codes of one unit are staged in LDS for the four waves,
+// double-buffered, while the next unit's codes and weights are in flight.  In
+// the MFMA's lane layout (A row and B column = lane % 16, C rows 4 (lane / 16)
+// + i of column lane % 16) each lane holds one weight row, so its scales are
+// decoded once per unit.
 #include <math.h>
 
 #include "cpv_internal.h"
@@ -33,9 +28,17 @@ namespace {
 constexpr int WBM = 64;                 // activation rows per workgroup
 constexpr int WT = 256;                 // threads per workgroup (4 waves)
 constexpr int WROW = 256 + 16;          // LDS bytes per staged activation row (+16 spreads the banks)
+constexpr int MAX_NMT = 8;              // 16-row activation blocks per workgroup (K-quants)
+// workgroups per CU: three waves per SIMD hold 168 registers, up to two blocks
+constexpr int wide_per_cu(int nmt) { return nmt > 2 ? 2 : 3; }
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v2i __attribute__((ext_vector_type(2)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef unsigned short v2u __attribute__((ext_vector_type(2)));
 
 struct WideArgs {
     const uint8_t* w;      // repacked Q4_K tiles: [tile][unit][9 pieces][64 rows][16 B]
@@ -46,6 +49,10 @@ struct WideArgs {
     int64_t n_pad;
     int U, M, m0, win;
     int tiles, mblocks, ksplit, upk;   // grid = tiles * mblocks * ksplit; upk units per K slice
+    const int32_t* bs16;   // [rows][U*16] sums of 16 codes (Q8_K)
+    float* y;              // outputs [rows][n], or null: the sums stay in gsum
+    int64_t n;             // weight rows
+    int nfull;             // (tile, row block) pairs that run over all of K
 };
 
 __device__ __forceinline__ int64_t pack2(uint32_t lo, uint32_t hi)
@@ -58,82 +65,211 @@ __device__ __forceinline__ v4i mfma16(int64_t a, int64_t b, v4i c)
     return __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b, c, 0, 0, 0);
 }
 
-__device__ __forceinline__ int byte_at(uint32_t w, int i) { return (int)((w >> (8 * i)) & 0xffu); }
+struct WidePart { int pair, u0, u1; bool whole; };
 
-// NMT: 16-row blocks of the 64 that hold rows (fewer when M <= 48)
-template <int NMT>
-__global__ __launch_bounds__(WT) __attribute__((amdgpu_waves_per_eu(3))) void qgemm_wide_kernel(WideArgs a)
+// workgroup -> (tile, row block) pair and its units.  Pairs 0 .. nfull - 1 run
+// whole; each later one in a.ksplit slices of a.upk units.  Consecutive
+// workgroups go to different XCDs, so the order is laid out per XCD: the row
+// blocks of one tile (which read the same weights) run side by side on one
+// XCD's L2.
+__device__ __forceinline__ WidePart wide_part(const WideArgs& a, int b)
 {
-    __shared__ __align__(16) uint8_t s_codes[2][16 * NMT][WROW];
-    __shared__ double s_dad[2][16 * NMT + 1];   // da * 2^(win - Ea) per staged row (+ a dump slot)
-    __shared__ double s_sm[WBM];        // 2^(win - Ea(m)), 0 for an all-zero row
+    WidePart p;
+    if (b < a.nfull) {
+        p.pair = (a.nfull & 7) == 0 ? (b & 7) * (a.nfull >> 3) + (b >> 3) : b;
+        p.u0 = 0;
+        p.u1 = a.U;
+        p.whole = true;
+        return p;
+    }
+    const int rest = (int)gridDim.x - a.nfull, c = b - a.nfull;
+    const int l = (rest & 7) == 0 ? (c & 7) * (rest >> 3) + (c >> 3) : c;
+    // (slices of the row blocks of a tile side by side)
+    const int np = rest / a.ksplit, ks = l / np;
+    p.pair = a.nfull + (l - ks * np);
+    p.u0 = ks * a.upk;
+    p.u1 = min(a.U, p.u0 + a.upk);
+    p.whole = a.ksplit == 1;
+    return p;
+}
+
+// Ea(m) of the block's 16 NMT rows: the exponent of the row's largest |scale|
+// (several lanes a row, so that a row's loads are in flight together)
+template <int NMT>
+__device__ __forceinline__ void wide_row_exponents(const WideArgs& a, int rbase, int nda, double* s_sm, int* s_ea)
+{
+    constexpr int R = 16 * NMT, TPR = NMT > 4 ? 2 : NMT > 2 ? 4 : NMT > 1 ? 8 : 16;
+    const int r = threadIdx.x / TPR, sub = threadIdx.x % TPR;
+    const float* d = a.da + (int64_t)min(rbase + (r < R ? r : R - 1), a.M - 1) * nda;
+    float mx = 0.0f;
+#pragma unroll 8
+    for (int u = sub; u < nda; u += TPR) mx = fmaxf(mx, fabsf(d[u]));
+    mx = cpv_group_reduce<TPR>(mx, cpv_op_max());
+    if (sub == 0 && r < R) {
+        const int e = cpv_exp_of_max(mx);
+        s_ea[r] = e;
+        s_sm[r] = e == CPV_E_EMPTY ? 0.0 : ldexp(1.0, a.win - e);
+    }
+}
+
+// the block's sums: outputs directly when y is asked for and the workgroup
+// covers all of K; else stored in the accumulator (whole) or added to it
+template <int NMT>
+__device__ __forceinline__ void wide_store(const WideArgs& a, const WidePart& wp, int tile, int rbase, int nrow, int g,
+                                           int er, const int* s_ea, const double (&S)[NMT][4])
+{
+    const int64_t n = (int64_t)tile * 64 + nrow;
+#pragma unroll
+    for (int mt = 0; mt < NMT; mt++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int r = mt * 16 + 4 * g + i, m = rbase + r;
+            if (m >= a.M) continue;
+            if (a.y && wp.whole) {
+                if (n < a.n) a.y[(int64_t)m * a.n + n] = cpv_gout_value(S[mt][i], er, s_ea[r], a.win);
+            } else {
+                double* p = a.gsum + (int64_t)m * a.n_pad + n;
+                if (wp.whole) *p = S[mt][i];
+                else unsafeAtomicAdd(p, S[mt][i]);
+            }
+        }
+}
+
+// the outputs of the sliced pairs (from a.nfull on): y from the accumulator,
+// which is left zero.  One workgroup per pair and 16-row block.
+__global__ __launch_bounds__(WT) void wide_finalize_kernel(WideArgs a, int nda, int rows)
+{
+    const int pair = a.nfull + blockIdx.x, tile = pair / a.mblocks, mb = pair - tile * a.mblocks;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t n = (int64_t)tile * 64 + lane;
+    const int e = a.ew[n];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int m = mb * rows + blockIdx.y * 16 + wave + 4 * q;
+        const int mc = min(m, a.M - 1);
+        float mx = 0.0f;
+        for (int u = lane; u < nda; u += 64) mx = fmaxf(mx, fabsf(a.da[(int64_t)mc * nda + u]));
+        mx = cpv_wave_reduce(mx, cpv_op_max());
+        if (m >= a.M) continue;
+        double* p = a.gsum + (int64_t)m * a.n_pad + n;
+        const double S = *p;
+        *p = 0.0;
+        if (n < a.n) a.y[(int64_t)m * a.n + n] = cpv_gout_value(S, e, cpv_exp_of_max(mx), a.win);
+    }
+}
+
+// ---------------------------------------------------------------- Q4_K and Q6_K
+// What bounds these kernels is VALU issue: per 16 x 16 outputs and unit the
+// contract's binary64 terms cost 40 instructions (Q4_K; 20 for Q6_K) at about
+// 2.1 ns each, and an int8 MFMA takes two of those issue slots and 7 ns of its
+// pipe whether it is 32 or 64 deep.  So everything else is made rare:
+//  * the sub-block scales enter through the B operands.  Q4_K: a code times
+//    the low (high) 3 bits of its scale is at most 15 * 7 = 105, so isum =
+//    8 * (codes * high . a) + (codes * low . a), two chains of four 16x16x64
+//    MFMAs, where 32-deep MFMAs per sub-block need 8 and a multiply-add per
+//    output and sub-block.  Q6_K: code * scale (13 bits signed) as two signed
+//    bytes, isum = 256 * high + low.  The bytes are built once per unit and
+//    wave (75 instructions, Q6_K about 210) and meet up to 8 row blocks.
+//  * Q4_K's imin = sum over the unit's 16-code groups of mn_j * (group sum) is
+//    one 16x16x16 f16 MFMA on the quantizer's group sums: mn <= 63 and |sum|
+//    <= 2032 are f16 values, every partial sum an integer below 2^21.
+//  * a lane loads whole 16-byte weight pieces: MFMA k of a unit takes its k
+//    slots from the pieces g and g + 4 of lane group g = lane / 16 (the
+//    reduction runs in any order; the activations are read in the same one).
+//  * activation codes go from memory to LDS without passing registers.
+//  * one block's binary64 terms run beside the next block's MFMAs.
+//  * outputs leave the kernel directly where it covers all of K.
+// 17408 x 5120 at 256 rows, whole call: Q4_K 141 -> 94 us, Q6_K 210 -> 85;
+// at 64 rows 62 -> 45 and 77 -> 49.
+template <int TYPE, int NMT>
+struct KqLds {
+    static constexpr int R = 16 * NMT;
+    static constexpr bool MIN = TYPE == CPV_Q4_K;
+    uint8_t codes[2][R][256];            // 16-byte piece p of row r at slot p ^ (r % 16)
+    double dad[2][R];                    // da * 2^(win - Ea) per staged row
+    double sm[R];                        // 2^(win - Ea(m)), 0 for an all-zero row
+    _Float16 bs[MIN ? 2 : 1][MIN ? R : 1][16];   // the group sums (exact in f16)
+};
+
+template <int TYPE, int NMT>
+__global__ __launch_bounds__(WT) __attribute__((amdgpu_waves_per_eu(wide_per_cu(NMT)))) void qgemm_wide_kq_kernel(WideArgs a)
+{
+    constexpr bool Q4 = TYPE == CPV_Q4_K;
+    constexpr int R = 16 * NMT, PCS = Q4 ? 9 : 13;
+    __shared__ __align__(16) KqLds<TYPE, NMT> s;
+    __shared__ int s_ea[R];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int U = a.U, M = a.M;
     const int64_t Kp = (int64_t)U * 256;
+    const WidePart wp = wide_part(a, blockIdx.x);
+    const int tile = wp.pair / a.mblocks, rbase = (wp.pair - tile * a.mblocks) * R, u0 = wp.u0, u1 = wp.u1;
 
-    // workgroup -> (tile, K slice, row block).  Consecutive workgroups go to
-    // different XCDs, so the order is laid out per XCD: the row blocks of one
-    // tile (which read the same weights) run side by side on one XCD's L2.
-    const int nb = gridDim.x, b0 = blockIdx.x;
-    const int L = (nb & 7) == 0 ? (b0 & 7) * (nb >> 3) + (b0 >> 3) : b0;
-    const int mb = L % a.mblocks, r0 = L / a.mblocks;
-    const int ks = r0 % a.ksplit, tile = r0 / a.ksplit;
-    const int u0 = ks * a.upk, u1 = min(U, u0 + a.upk);
-    const int rbase = mb * WBM;
+    wide_row_exponents<NMT>(a, rbase, U, s.sm, s_ea);
 
-    // Ea(m) per row of the block: the exponent of the row's largest |scale|
-    for (int r = wave; r < WBM; r += WT / 64) {
-        const int mr = a.m0 + min(rbase + r, M - 1);
-        float mx = 0.0f;
-        for (int u = lane; u < U; u += 64) mx = fmaxf(mx, fabsf(a.da[(int64_t)mr * U + u]));
-        mx = cpv_wave_reduce(mx, cpv_op_max());
-        if (lane == 0) {
-            int e = CPV_E_EMPTY;
-            if (mx > 0.0f) frexpf(mx, &e);
-            s_sm[r] = e == CPV_E_EMPTY ? 0.0 : ldexp(1.0, a.win - e);
+    // staging of one unit: the codes go from memory into LDS directly, 4 rows
+    // per wave and load (LDS slot = lane, so the swizzle is in the source
+    // address); the row scales and (Q4_K) the rows' 16 group sums, 8 per
+    // thread, pass through registers.  Surplus threads repeat another's row
+    // (the same values to the same place: no branch)
+    int soff[NMT];
+#pragma unroll
+    for (int q = 0; q < NMT; q++) {
+        const int r = (q * 4 + wave) * 4 + (lane >> 4);
+        soff[q] = (min(rbase + r, M - 1) - rbase) * (int)Kp + ((lane & 15) ^ (r & 15)) * 16;
+    }
+    const int8_t* qbase = a.qa + (int64_t)rbase * Kp;
+    const int drow = tid % R, brow = (tid >> 1) % R;
+    const float* sda = a.da + (int64_t)min(rbase + drow, M - 1) * U;
+    const int32_t* sbs = a.bs16 + (int64_t)min(rbase + brow, M - 1) * U * 16 + 8 * (tid & 1);
+    struct Stage { v4i b[Q4 ? 2 : 1]; float d; };
+    auto stage_load = [&](int u, int buf, Stage& t) {
+#pragma unroll
+        for (int q = 0; q < NMT; q++)
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(qbase + soff[q] + u * 256),
+                                             (__attribute__((address_space(3))) void*)&s.codes[buf][(q * 4 + wave) * 4][0],
+                                             16, 0, 0);
+        if constexpr (Q4) {
+            t.b[0] = *(const v4i*)(sbs + u * 16);
+            t.b[1] = *(const v4i*)(sbs + u * 16 + 4);
         }
-    }
-
-    // staging of one unit: 64 rows x 16 pieces of 16 B, 4 per thread, and the row scales
-    // (32-bit offsets from the block's first row: rows * Kp stays below 2^31)
-    const int8_t* qbase = a.qa + (int64_t)(a.m0 + rbase) * Kp;
-    int soff[4];
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const int p = tid + q * WT, r = p >> 4;
-        soff[q] = (min(rbase + r, M - 1) - rbase) * (int)Kp + (p & 15) * 16;
-    }
-    const float* sda = a.da + (int64_t)(a.m0 + min(rbase + (tid & 63), M - 1)) * U;
-    auto stage_load = [&](int u, v4i* cv, float& dv) {
-#pragma unroll
-        for (int q = 0; q < NMT; q++) cv[q] = *(const v4i*)(qbase + soff[q] + u * 256);
-        dv = sda[u];
+        t.d = sda[u];
     };
-    auto stage_store = [&](int buf, const v4i* cv, float dv) {
+    auto stage_store = [&](int buf, const Stage& t) {
+        if constexpr (Q4) {
+            v8h h;
 #pragma unroll
-        for (int q = 0; q < NMT; q++) {
-            const int p = tid + q * WT;
-            *(v4i*)&s_codes[buf][p >> 4][(p & 15) * 16] = cv[q];
+            for (int i = 0; i < 8; i++) h[i] = (_Float16)(float)t.b[i >> 2][i & 3];
+            *(v8h*)&s.bs[buf][brow][8 * (tid & 1)] = h;
         }
-        // (threads past the rows write the dump slot: no branch around the store)
-        const int sr = tid < 16 * NMT ? tid : 16 * NMT;
-        s_dad[buf][sr] = (double)dv * s_sm[tid & (WBM - 1)];
+        s.dad[buf][drow] = (double)t.d * s.sm[drow];
     };
 
-    // this lane's weight row and k slot: 8 codes (bytes 8 (kq & 1).. of piece
-    // (pr, kq >> 1)) per 64-element chunk pr, and the row's scale piece
-    const int nl = lane & 15, kq = lane >> 4;
+    // this lane's weight row, its pieces g and g + 4 of the codes (and for
+    // Q6_K the pieces of the high bits beside them) and the scale piece
+    const int nl = lane & 15, g = lane >> 4;
     const int nrow = wave * 16 + nl;
-    const uint8_t* wrow = a.w + (int64_t)tile * U * 9 * 1024 + nrow * 16;
-    struct Wt { v2i q[4]; v4i s; };
+    const uint8_t* wrow = a.w + (int64_t)tile * U * PCS * 1024 + nrow * 16;
+    const uint16_t* wd = (const uint16_t*)(a.w + (int64_t)(a.n_pad / 64) * U * 13 * 1024) + (int64_t)tile * U * 64 + nrow;
+    struct Wt { v4i q[2]; v4i h[Q4 ? 1 : 2]; v4i s; uint32_t d; };
     auto wload = [&](int u, Wt& t) {
-        const uint8_t* p = wrow + (int64_t)u * 9 * 1024;
-#pragma unroll
-        for (int pr = 0; pr < 4; pr++) t.q[pr] = *(const v2i*)(p + (2 * pr + (kq >> 1)) * 1024 + 8 * (kq & 1));
-        t.s = *(const v4i*)(p + 8 * 1024);
+        const uint8_t* p = wrow + (int64_t)u * PCS * 1024;
+        t.q[0] = *(const v4i*)(p + g * 1024);
+        t.q[1] = *(const v4i*)(p + (4 + g) * 1024);
+        if constexpr (!Q4) {
+            t.h[0] = *(const v4i*)(p + (8 + (g & 1)) * 1024);
+            t.h[1] = *(const v4i*)(p + (10 + (g & 1)) * 1024);
+            t.d = wd[(int64_t)u * 64];
+        }
+        t.s = *(const v4i*)(p + (PCS - 1) * 1024);
     };
     const int er = a.ew[(int64_t)tile * 64 + nrow];
+    // the activations of MFMA k: piece 8 (k >> 1) + (Q4_K: 2, Q6_K: 4) (k & 1)
+    // above the lane group's, at its swizzled slot
+    int aoff[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        aoff[k] = nl * 256 + (((Q4 ? 4 * (g >> 1) + (g & 1) : g) + 8 * (k >> 1) + (Q4 ? 2 : 4) * (k & 1)) ^ nl) * 16;
 
     double S[NMT][4];
 #pragma unroll
@@ -142,91 +278,149 @@ __global__ __launch_bounds__(WT) __attribute__((amdgpu_waves_per_eu(3))) void qg
         for (int i = 0; i < 4; i++) S[mt][i] = 0.0;
 
     Wt wc, wn;
-    v4i cv[NMT];
-    float dv;
+    Stage st;
     wload(u0, wc);
-    stage_load(u0, cv, dv);
-    __syncthreads();                    // s_sm
-    stage_store(0, cv, dv);
+    stage_load(u0, 0, st);
+    __syncthreads();                     // s.sm
+    stage_store(0, st);
     __syncthreads();
 
     for (int u = u0; u < u1; u++) {
         const int buf = (u - u0) & 1;
-        // the next unit in flight (the last one reloads itself: no branch)
-        const int un = u + 1 < u1 ? u + 1 : u;
+        const int un = u + 1 < u1 ? u + 1 : u;   // (the last one reloads itself: no branch)
         wload(un, wn);
-        stage_load(un, cv, dv);
+        stage_load(un, buf ^ 1, st);
 
-        // this unit's scales and B operands
-        const uint32_t h0 = (uint32_t)wc.s[0], hy = (uint32_t)wc.s[1], hz = (uint32_t)wc.s[2],
-                       hw = (uint32_t)wc.s[3];
-        const double dws = ldexp((double)cpv_h2f((uint16_t)(h0 & 0xffffu)), -er);
-        const double dms = ldexp((double)cpv_h2f((uint16_t)(h0 >> 16)), -er);
-        const uint32_t sc_lo = hy & 0x3f3f3f3fu, mn_lo = hz & 0x3f3f3f3fu;
-        const uint32_t sc_hi = (hw & 0x0f0f0f0fu) | (((hy >> 6) & 0x03030303u) << 4);
-        const uint32_t mn_hi = ((hw >> 4) & 0x0f0f0f0fu) | (((hz >> 6) & 0x03030303u) << 4);
-        // per sub-block j: its B operands (codes, mn_j in every byte) built here, then
-        // the four 16-row blocks; the dots are scaled by sc_j as they come
-        int isum[NMT][4];
-        v4i dmin[NMT];
+        // B operands of the unit's four 64-deep steps: high and low limbs
+        v4i bh[4], bl[4];
+        v4h bm;
+        double dws, dms = 0.0;
+        if constexpr (Q4) {
+            const uint32_t h0 = (uint32_t)wc.s[0], hy = (uint32_t)wc.s[1], hz = (uint32_t)wc.s[2], hw = (uint32_t)wc.s[3];
+            dws = ldexp((double)cpv_h2f((uint16_t)(h0 & 0xffffu)), -er);
+            dms = ldexp((double)cpv_h2f((uint16_t)(h0 >> 16)), -er);
+            // scales and mins of sub-blocks 0-3 and 4-7; this lane's are 2 (g >> 1), + 1 of each four
+            const uint32_t sc[2] = {hy & 0x3f3f3f3fu, (hw & 0x0f0f0f0fu) | ((hy >> 2) & 0x30303030u)};
+            const uint32_t mlo = hz & 0x3f3f3f3fu, mhi = ((hw >> 4) & 0x0f0f0f0fu) | ((hz >> 2) & 0x30303030u);
 #pragma unroll
-        for (int mt = 0; mt < NMT; mt++) {
-            dmin[mt] = v4i{0, 0, 0, 0};
+            for (int hf = 0; hf < 2; hf++) {
+                const uint32_t sl = sc[hf] & 0x07070707u, sh = (sc[hf] >> 3) & 0x07070707u;
 #pragma unroll
-            for (int i = 0; i < 4; i++) isum[mt][i] = 0;
-        }
+                for (int nb = 0; nb < 2; nb++) {
+                    // the sub-block's byte in both 16-bit halves
+                    const uint32_t sel = (g >> 1) ? (nb ? 0x0c030c03u : 0x0c020c02u) : (nb ? 0x0c010c01u : 0x0c000c00u);
+                    const v2u ml = __builtin_bit_cast(v2u, __builtin_amdgcn_perm(sl, sl, sel));
+                    const v2u mh = __builtin_bit_cast(v2u, __builtin_amdgcn_perm(sh, sh, sel));
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const uint32_t x0 = (uint32_t)wc.q[j >> 1][0], x1 = (uint32_t)wc.q[j >> 1][1];
-            const int sh = 4 * (j & 1);   // sub-block 2 pr: low nibbles, 2 pr + 1: high
-            const int64_t bq = pack2((x0 >> sh) & 0x0f0f0f0fu, (x1 >> sh) & 0x0f0f0f0fu);
-            const uint32_t mw = j < 4 ? mn_lo : mn_hi;
-            const uint32_t bb = __builtin_amdgcn_perm(mw, mw, (uint32_t)(j & 3) * 0x01010101u);
-            const int64_t bm = pack2(bb, bb);
-            const int scj = byte_at(j < 4 ? sc_lo : sc_hi, j & 3);
-#pragma unroll
-            for (int mt = 0; mt < NMT; mt++) {
-                const int64_t av = *(const int64_t*)&s_codes[buf][mt * 16 + nl][8 * kq + 32 * j];
-                const v4i d = mfma16(av, bq, v4i{0, 0, 0, 0});
-                dmin[mt] = mfma16(av, bm, dmin[mt]);
-#pragma unroll
-                for (int i = 0; i < 4; i++) isum[mt][i] += __mul24(scj, d[i]);   // |dot| <= 32*15*127
+                    for (int x = 0; x < 4; x++) {
+                        const uint32_t w = (uint32_t)wc.q[hf][x];
+                        const v2u c = __builtin_bit_cast(v2u, (nb ? w >> 4 : w) & 0x0f0f0f0fu);
+                        bl[2 * hf + nb][x] = __builtin_bit_cast(int, c * ml);   // (bytes <= 105: no carry)
+                        bh[2 * hf + nb][x] = __builtin_bit_cast(int, c * mh);
+                    }
+                }
             }
-            // one sub-block at a time: the scaled dots are taken here (else the
-            // compiler sinks them and keeps all 32 MFMA results live, which
-            // costs the registers of a second wave per SIMD)
+            // mn of k slots 4 g .. 4 g + 3: the 16-code groups of sub-blocks 2 g and 2 g + 1
+            // (0x6400 | b is 1024 + b in f16)
+            const uint32_t mw = ((g >> 1) ? mhi : mlo) >> (16 * (g & 1));
+            const uint32_t p0 = __builtin_amdgcn_perm(0x64646464u, mw, 0x04000400u);
+            const uint32_t p1 = __builtin_amdgcn_perm(0x64646464u, mw, 0x04010401u);
+            const v2h k1024 = {(_Float16)1024.0f, (_Float16)1024.0f};
+            const v2h m0 = __builtin_bit_cast(v2h, p0) - k1024, m1 = __builtin_bit_cast(v2h, p1) - k1024;
+            bm = v4h{m0[0], m0[1], m1[0], m1[1]};
+        } else {
+            dws = ldexp((double)cpv_h2f((uint16_t)wc.d), -er);
 #pragma unroll
-            for (int mt = 0; mt < NMT; mt++)
-                asm volatile("" : "+v"(isum[mt][0]), "+v"(isum[mt][1]), "+v"(isum[mt][2]), "+v"(isum[mt][3]));
-            __builtin_amdgcn_sched_barrier(0);
+            for (int hf = 0; hf < 2; hf++)
+#pragma unroll
+                for (int nb = 0; nb < 2; nb++) {
+                    // the 16-code group's scale; product + 128 per code, so that its
+                    // high byte is the high limb and its low byte the low limb + 128
+                    const int sc = (int)(int8_t)((uint32_t)wc.s[2 * hf + nb] >> (8 * g));
+                    const uint32_t su = (uint32_t)(sc & 0xffff), cu = (uint32_t)((128 - 32 * sc) & 0xffff);
+                    const v2u s2 = __builtin_bit_cast(v2u, su * 0x10001u), c2 = __builtin_bit_cast(v2u, cu | (cu << 16));
+                    const int qsh = 2 * (g >> 1) + 4 * nb;
+#pragma unroll
+                    for (int x = 0; x < 4; x++) {
+                        const uint32_t w = (uint32_t)wc.q[hf][x];
+                        const uint32_t q = ((nb ? w >> 4 : w) & 0x0f0f0f0fu) |
+                                           ((((uint32_t)wc.h[hf][x] >> qsh) & 0x03030303u) << 4);
+                        const v2u e = __builtin_bit_cast(v2u, q & 0x00ff00ffu), o = __builtin_bit_cast(v2u, (q >> 8) & 0x00ff00ffu);
+                        const uint32_t pe = __builtin_bit_cast(uint32_t, e * s2 + c2), po = __builtin_bit_cast(uint32_t, o * s2 + c2);
+                        bl[2 * hf + nb][x] = (int)(__builtin_amdgcn_perm(po, pe, 0x06020400u) ^ 0x80808080u);
+                        bh[2 * hf + nb][x] = (int)__builtin_amdgcn_perm(po, pe, 0x07030501u);
+                    }
+                }
         }
+        // block mt's binary64 terms run beside block mt + 1's MFMAs, whose A
+        // operands were read one block earlier
+        const uint8_t* cb = &s.codes[buf][0][0];
+        v4i av[4];
+        v4h ab;
+        struct Acc { v4i hi, lo; v4f mn; };
+        auto mma = [&](int mt, Acc& c, bool more) {
+            c.hi = c.lo = v4i{0, 0, 0, 0};
+            if constexpr (Q4) {
+                c.mn = __builtin_amdgcn_mfma_f32_16x16x16f16(ab, bm, v4f{0, 0, 0, 0}, 0, 0, 0);
+                if (more) ab = *(const v4h*)&s.bs[buf][(mt + 1) * 16 + nl][4 * g];
+            }
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                c.hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[k], bh[k], c.hi, 0, 0, 0);
+                c.lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[k], bl[k], c.lo, 0, 0, 0);
+                if (more) av[k] = *(const v4i*)(cb + aoff[k] + (mt + 1) * 4096);
+            }
+        };
+        struct Da { double v[4]; };
+        auto da_of = [&](int mt) {
+            Da d;
+#pragma unroll
+            for (int i = 0; i < 4; i++) d.v[i] = s.dad[buf][mt * 16 + 4 * g + i];
+            return d;
+        };
+        Acc c[2];
+#pragma unroll
+        for (int k = 0; k < 4; k++) av[k] = *(const v4i*)(cb + aoff[k]);
+        if constexpr (Q4) ab = *(const v4h*)&s.bs[buf][nl][4 * g];
+        mma(0, c[0], NMT > 1);
+        Da dc = da_of(0), dn = dc;
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int mt = 0; mt < NMT; mt++) {
-            const double* dd = &s_dad[buf][mt * 16 + 4 * kq];
+            if (mt + 1 < NMT) {
+                mma(mt + 1, c[(mt + 1) & 1], mt + 2 < NMT);
+                dn = da_of(mt + 1);
+            }
+            const Acc& x = c[mt & 1];
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const double da = dd[i];
-                S[mt][i] += rint(dws * da * (double)isum[mt][i]) - rint(dms * da * (double)dmin[mt][i]);
+                const double da = dc.v[i];
+                if constexpr (Q4) S[mt][i] += rint(dws * da * (double)(x.hi[i] * 8 + x.lo[i])) - rint(dms * da * (double)x.mn[i]);
+                else S[mt][i] += rint(dws * da * (double)(x.hi[i] * 256 + x.lo[i]));
             }
+            if (mt + 1 < NMT) {
+                if constexpr (Q4) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+                }
+                __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);       // the next block's group sums and row scales
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA
+                    __builtin_amdgcn_sched_group_barrier(0x002, Q4 ? 5 : 3, 0);   // VALU
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // LDS read
+                    __builtin_amdgcn_sched_group_barrier(0x002, Q4 ? 5 : 3, 0);
+                }
+            }
+            dc = dn;
+            __builtin_amdgcn_sched_barrier(0);
         }
-        stage_store(buf ^ 1, cv, dv);
+        stage_store(buf ^ 1, st);
         __syncthreads();
         wc = wn;
     }
-
-    // the sums: stored when this workgroup covers all of K, else added
-    double* g = a.gsum + (int64_t)tile * 64 + nrow;
-#pragma unroll
-    for (int mt = 0; mt < NMT; mt++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int m = rbase + mt * 16 + 4 * kq + i;
-            if (m < M) {
-                double* p = g + (int64_t)(a.m0 + m) * a.n_pad;
-                if (a.ksplit == 1) *p = S[mt][i];
-                else unsafeAtomicAdd(p, S[mt][i]);
-            }
-        }
+    wide_store<NMT>(a, wp, tile, rbase, nrow, g, er, s_ea, S);
 }
 
 // The same for Q8_0 weights and activations (ggml's Q8_0 vec_dot_type).
@@ -363,171 +557,6 @@ __global__ __launch_bounds__(WT) __attribute__((amdgpu_waves_per_eu(2))) void qg
         }
 }
 
-// The same for Q6_K weights (Q8_K activations).  Per (activation row m,
-// weight row n, unit) the integer isum = sum_g sc_g * dot_g over the 16
-// groups of 16 codes (q - 32), then one binary64 term rint(A * isum) as the
-// contract has it.  Per 32-element chunk c (half h = c / 4, quarter s = c %
-// 4) a lane's 8 codes are the low (s < 2) or high nibbles of ql bytes 64 h +
-// 32 (s & 1) + 8 kq .., with qh bits 2 s, 2 s + 1 of bytes 32 h + 8 kq ..
-// above them; the chunk's two groups go through two MFMAs whose B operands
-// hold the codes in the group's k slots (kq < 2, kq >= 2) and zeros in the
-// other's.  A unit's pieces: ql 0-7, qh 8-11, the 16 group scales 12; the
-// unit's d (f16) lies in a region of its own after the tiles.
-// NMT: 16-row blocks of the 64 that hold rows (fewer when M <= 48)
-template <int NMT>
-__global__ __launch_bounds__(WT) __attribute__((amdgpu_waves_per_eu(2))) void qgemm_wide_q6k_kernel(WideArgs a)
-{
-    __shared__ __align__(16) uint8_t s_codes[2][16 * NMT][WROW];
-    __shared__ double s_dad[2][16 * NMT];   // da * 2^(win - Ea) per staged row
-    __shared__ double s_sm[WBM];        // 2^(win - Ea(m)), 0 for an all-zero row
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int U = a.U, M = a.M;
-    const int64_t Kp = (int64_t)U * 256;
-
-    const int nb = gridDim.x, b0 = blockIdx.x;
-    const int L = (nb & 7) == 0 ? (b0 & 7) * (nb >> 3) + (b0 >> 3) : b0;
-    const int mb = L % a.mblocks, r0 = L / a.mblocks;
-    const int ks = r0 % a.ksplit, tile = r0 / a.ksplit;
-    const int u0 = ks * a.upk, u1 = min(U, u0 + a.upk);
-    const int rbase = mb * WBM;
-
-    for (int r = wave; r < WBM; r += WT / 64) {
-        const int mr = a.m0 + min(rbase + r, M - 1);
-        float mx = 0.0f;
-        for (int u = lane; u < U; u += 64) mx = fmaxf(mx, fabsf(a.da[(int64_t)mr * U + u]));
-        mx = cpv_wave_reduce(mx, cpv_op_max());
-        if (lane == 0) {
-            int e = CPV_E_EMPTY;
-            if (mx > 0.0f) frexpf(mx, &e);
-            s_sm[r] = e == CPV_E_EMPTY ? 0.0 : ldexp(1.0, a.win - e);
-        }
-    }
-
-    const int8_t* qbase = a.qa + (int64_t)(a.m0 + rbase) * Kp;
-    int soff[4];
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const int p = tid + q * WT, r = p >> 4;
-        soff[q] = (min(rbase + r, M - 1) - rbase) * (int)Kp + (p & 15) * 16;
-    }
-    const float* sda = a.da + (int64_t)(a.m0 + min(rbase + (tid & 63), M - 1)) * U;
-    auto stage_load = [&](int u, v4i* cv, float& dv) {
-#pragma unroll
-        for (int q = 0; q < NMT; q++) cv[q] = *(const v4i*)(qbase + soff[q] + u * 256);
-        dv = sda[u];
-    };
-    auto stage_store = [&](int buf, const v4i* cv, float dv) {
-#pragma unroll
-        for (int q = 0; q < NMT; q++) {
-            const int p = tid + q * WT;
-            *(v4i*)&s_codes[buf][p >> 4][(p & 15) * 16] = cv[q];
-        }
-        if (tid < 16 * NMT) s_dad[buf][tid] = (double)dv * s_sm[tid];
-    };
-
-    const int nl = lane & 15, kq = lane >> 4;
-    const int nrow = wave * 16 + nl;
-    const uint8_t* wrow = a.w + (int64_t)tile * U * 13 * 1024 + nrow * 16;
-    const uint16_t* drow = (const uint16_t*)(a.w + (int64_t)(a.n_pad / 64) * U * 13 * 1024) + (int64_t)tile * U * 64 + nrow;
-    struct Wt { v2i ql[2][2]; v2i qh[2]; v4i s; uint32_t d; };
-    auto wload = [&](int u, Wt& t) {
-        const uint8_t* p = wrow + (int64_t)u * 13 * 1024 + 8 * (kq & 1);
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-#pragma unroll
-            for (int s1 = 0; s1 < 2; s1++) t.ql[h][s1] = *(const v2i*)(p + (4 * h + 2 * s1 + (kq >> 1)) * 1024);
-            t.qh[h] = *(const v2i*)(p + (8 + 2 * h + (kq >> 1)) * 1024);
-        }
-        t.s = *(const v4i*)(wrow + (int64_t)u * 13 * 1024 + 12 * 1024);
-        t.d = drow[(int64_t)u * 64];
-    };
-    const int er = a.ew[(int64_t)tile * 64 + nrow];
-    // the 4 codes of a dword as signed bytes q - 32 (q in 0..63: q ^ 32,
-    // with bits 6 and 7 set where q < 32)
-    auto centered = [](uint32_t q) {
-        const uint32_t t = q ^ 0x20202020u;
-        return t | (((t >> 5) & 0x01010101u) * 0xc0u);
-    };
-
-    double S[NMT][4];
-#pragma unroll
-    for (int mt = 0; mt < NMT; mt++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) S[mt][i] = 0.0;
-
-    Wt wc, wn;
-    v4i cv[NMT];
-    float dv;
-    wload(u0, wc);
-    stage_load(u0, cv, dv);
-    __syncthreads();                    // s_sm
-    stage_store(0, cv, dv);
-    __syncthreads();
-
-    for (int u = u0; u < u1; u++) {
-        const int buf = (u - u0) & 1;
-        const int un = u + 1 < u1 ? u + 1 : u;
-        wload(un, wn);
-        stage_load(un, cv, dv);
-        const double dws = ldexp((double)cpv_h2f((uint16_t)wc.d), -er);
-        int isum[NMT][4];
-#pragma unroll
-        for (int mt = 0; mt < NMT; mt++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) isum[mt][i] = 0;
-#pragma unroll
-        for (int c = 0; c < 8; c++) {
-            const int h = c >> 2, sq = c & 3;
-            uint32_t cw[2];
-#pragma unroll
-            for (int x = 0; x < 2; x++) {
-                const uint32_t lo = ((uint32_t)wc.ql[h][sq & 1][x] >> (4 * (sq >> 1))) & 0x0f0f0f0fu;
-                const uint32_t hi = (((uint32_t)wc.qh[h][x] >> (2 * sq)) & 0x03030303u) << 4;
-                cw[x] = centered(lo | hi);
-            }
-            const int64_t bc = pack2(cw[0], cw[1]);
-            const int64_t b0v = kq < 2 ? bc : 0, b1v = kq < 2 ? 0 : bc;   // group 2c, group 2c + 1
-            const uint32_t sw = (uint32_t)wc.s[c >> 1];
-            const int sc0 = (int)(int8_t)(sw >> (16 * (c & 1))), sc1 = (int)(int8_t)(sw >> (16 * (c & 1) + 8));
-#pragma unroll
-            for (int mt = 0; mt < NMT; mt++) {
-                const int64_t av = *(const int64_t*)&s_codes[buf][mt * 16 + nl][8 * kq + 32 * c];
-                const v4i d0 = mfma16(av, b0v, v4i{0, 0, 0, 0});
-                const v4i d1 = mfma16(av, b1v, v4i{0, 0, 0, 0});
-#pragma unroll
-                for (int i = 0; i < 4; i++) isum[mt][i] += sc0 * d0[i] + sc1 * d1[i];   // |isum| < 2^28
-            }
-#pragma unroll
-            for (int mt = 0; mt < NMT; mt++)
-                asm volatile("" : "+v"(isum[mt][0]), "+v"(isum[mt][1]), "+v"(isum[mt][2]), "+v"(isum[mt][3]));
-            __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int mt = 0; mt < NMT; mt++) {
-            const double* dd = &s_dad[buf][mt * 16 + 4 * kq];
-#pragma unroll
-            for (int i = 0; i < 4; i++) S[mt][i] += rint(dws * dd[i] * (double)isum[mt][i]);
-        }
-        stage_store(buf ^ 1, cv, dv);
-        __syncthreads();
-        wc = wn;
-    }
-
-    double* g = a.gsum + (int64_t)tile * 64 + nrow;
-#pragma unroll
-    for (int mt = 0; mt < NMT; mt++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int m = rbase + mt * 16 + 4 * kq + i;
-            if (m < M) {
-                double* p = g + (int64_t)(a.m0 + m) * a.n_pad;
-                if (a.ksplit == 1) *p = S[mt][i];
-                else unsafeAtomicAdd(p, S[mt][i]);
-            }
-        }
-}
-
 }  // namespace
 
 bool cpv_qgemm_wide_ok(const cpv_weight* w, int64_t m)
@@ -539,13 +568,74 @@ bool cpv_qgemm_wide_ok(const cpv_weight* w, int64_t m)
     return (w->type == CPV_Q4_K && m > 16) || ((w->type == CPV_Q6_K || w->type == CPV_Q8_0) && m > 8);
 }
 
-cpv_status cpv_qgemm_wide(cpv_ctx* ctx, const cpv_weight* w, const cpv_act* act, double* gsum, int win)
+namespace {
+
+// Rows per workgroup and the deal of the (tile, row block) pairs over the
+// chip's slots (workgroups in flight).  Whole rounds of pairs run over all of
+// K; the pairs that are left run in ks K slices of at least 4 units each.
+// Chosen by an estimate in us, from gate|up (17408 and 34816 x 5120), wo and
+// down (5120 x 5120, 5120 x 17408) at 128 to 256 rows: a unit takes 0.7 +
+// 0.335 nmt with the CU full and 0.62 of that with one workgroup on it, a
+// workgroup's start (row exponents, first loads) 3, and a million atomic adds
+// of a slice's sums 3.5 (they bypass the XCD's L2).  E.g. 17408 x 5120 at 128
+// rows: 8 blocks in 272 pairs 76 us a call, 4 in 544 pairs 62; 5120 x 17408 at
+// 256 rows: 8 blocks in 160 pairs x 3 slices 116, 4 in 320 whole pairs 146.
+void wide_split(WideArgs& a, int cus, int* nmt_out)
+{
+    const int nb16 = (a.M + 15) / 16;
+    double best = 1e30;
+    for (int mb = (nb16 + MAX_NMT - 1) / MAX_NMT; mb <= nb16; mb++) {
+        const int nmt = (nb16 + mb - 1) / mb;
+        if ((nb16 + nmt - 1) / nmt != mb) continue;   // (the same blocks in fewer workgroups)
+        const int slots = cus * wide_per_cu(nmt);
+        const int64_t pairs = (int64_t)a.tiles * mb, full = pairs / slots * slots, rest = pairs - full;
+        const double t = (0.7 + 0.335 * nmt) * wide_per_cu(nmt) / 2, t1 = 0.62 * t, s0 = 3.0;
+        const double tf = (double)(full / slots) * (a.U * t + s0);
+        for (int ks = 1; ks == 1 || (rest && ks <= a.U / 4 && ks <= 16); ks++) {
+            const int upk = (a.U + ks - 1) / ks, k2 = (a.U + upk - 1) / upk;
+            if (k2 != ks) continue;
+            const int64_t w = rest * ks, last = w % slots;
+            double tr = (double)(w / slots) * (upk * t + s0);
+            // (one workgroup a CU up to cus, then a share of the CUs full)
+            if (last) tr += upk * (last > cus ? t1 + (t - t1) * (double)(last - cus) / (slots - cus) : t1) + s0;
+            if (ks > 1) tr += (double)w * nmt * 1024 * 3.5e-6 + 1.5;
+            if (tf + tr < best) {
+                best = tf + tr;
+                *nmt_out = nmt;
+                a.mblocks = mb;
+                a.nfull = (int)(ks > 1 ? full : pairs);
+                a.ksplit = ks;
+                a.upk = upk;
+            }
+        }
+        if (nmt <= 2) break;
+    }
+}
+
+template <int TYPE>
+void kq_launch(const WideArgs& a, int nmt, unsigned grid, hipStream_t stream)
+{
+    switch (nmt) {
+    case 1: qgemm_wide_kq_kernel<TYPE, 1><<<grid, WT, 0, stream>>>(a); break;
+    case 2: qgemm_wide_kq_kernel<TYPE, 2><<<grid, WT, 0, stream>>>(a); break;
+    case 3: qgemm_wide_kq_kernel<TYPE, 3><<<grid, WT, 0, stream>>>(a); break;
+    case 4: qgemm_wide_kq_kernel<TYPE, 4><<<grid, WT, 0, stream>>>(a); break;
+    case 5: qgemm_wide_kq_kernel<TYPE, 5><<<grid, WT, 0, stream>>>(a); break;
+    case 6: qgemm_wide_kq_kernel<TYPE, 6><<<grid, WT, 0, stream>>>(a); break;
+    case 7: qgemm_wide_kq_kernel<TYPE, 7><<<grid, WT, 0, stream>>>(a); break;
+    default: qgemm_wide_kq_kernel<TYPE, 8><<<grid, WT, 0, stream>>>(a); break;
+    }
+}
+
+}  // namespace
+
+cpv_status cpv_qgemm_wide(cpv_ctx* ctx, const cpv_weight* w, const cpv_act* act, double* gsum, int win, float* y)
 {
     const bool q80 = w->type == CPV_Q8_0, q6k = w->type == CPV_Q6_K;
     if ((w->type != CPV_Q4_K && !q80 && !q6k) || act->kq == q80 || act->U != (int)w->units || act->m < 1 ||
         act->m > INT32_MAX / 2)
         return cpv_fail(ctx, CPV_EINVAL, "qgemm_wide: weight or activation format not supported");
-    if ((int64_t)WBM * act->U * 256 > INT32_MAX)   // the staging offsets within a row block are 32-bit
+    if (2LL * WBM * act->U * 256 > INT32_MAX)   // the staging offsets within a row block are 32-bit
         return cpv_fail(ctx, CPV_EUNSUPPORTED, "qgemm_wide: k=%lld too long", (long long)w->k);
     WideArgs a;
     a.w = (const uint8_t*)w->data;
@@ -559,26 +649,36 @@ cpv_status cpv_qgemm_wide(cpv_ctx* ctx, const cpv_weight* w, const cpv_act* act,
     a.m0 = 0;
     a.win = win;
     a.tiles = (int)(w->n_pad / 64);
-    a.mblocks = (a.M + WBM - 1) / WBM;
-    // slice K when the grid would leave CUs idle (about 3 workgroups fit a CU)
-    const int64_t blocks = (int64_t)a.tiles * a.mblocks, want = 3LL * ctx->cu_count;
-    int ksplit = blocks >= want ? 1 : (int)((want + blocks - 1) / blocks);
-    if (ksplit > a.U / 4) ksplit = a.U / 4 > 1 ? a.U / 4 : 1;
-    a.upk = (a.U + ksplit - 1) / ksplit;
-    a.ksplit = (a.U + a.upk - 1) / a.upk;
-    const int64_t grid = blocks * a.ksplit;
-    if (grid > INT32_MAX) return cpv_fail(ctx, CPV_EUNSUPPORTED, "qgemm_wide: grid of %lld", (long long)grid);
+    a.bs16 = act->bs16;
+    a.y = y;
+    a.n = w->n;
+    if ((int64_t)a.tiles * ((a.M + 15) / 16) > INT32_MAX / 1024)
+        return cpv_fail(ctx, CPV_EUNSUPPORTED, "qgemm_wide: %d tiles by %d rows", a.tiles, a.M);
+    int nmt = 4;
+    if (q80) {
+        // slice K when the grid would leave CUs idle (about 3 workgroups fit a CU)
+        a.mblocks = (a.M + WBM - 1) / WBM;
+        const int64_t blocks = (int64_t)a.tiles * a.mblocks, want = 3LL * ctx->cu_count;
+        int ksplit = blocks >= want ? 1 : (int)((want + blocks - 1) / blocks);
+        if (ksplit > a.U / 4) ksplit = a.U / 4 > 1 ? a.U / 4 : 1;
+        a.upk = (a.U + ksplit - 1) / ksplit;
+        a.ksplit = (a.U + a.upk - 1) / a.upk;
+        a.nfull = 0;
+    } else {
+        wide_split(a, ctx->cu_count, &nmt);
+    }
+    const int64_t blocks = (int64_t)a.tiles * a.mblocks;
+    const int64_t rest = blocks - a.nfull, grid = a.nfull + rest * a.ksplit;
     const int ev = cpv_prof_mark(ctx);
     auto go = [=]() {
         if (q80 && a.M <= 16) qgemm_wide_q80_kernel<1><<<(unsigned)grid, WT, 0, ctx->stream>>>(a);
         else if (q80 && a.M <= 32) qgemm_wide_q80_kernel<2><<<(unsigned)grid, WT, 0, ctx->stream>>>(a);
         else if (q80) qgemm_wide_q80_kernel<4><<<(unsigned)grid, WT, 0, ctx->stream>>>(a);
-        else if (q6k && a.M <= 16) qgemm_wide_q6k_kernel<1><<<(unsigned)grid, WT, 0, ctx->stream>>>(a);
-        else if (q6k && a.M <= 32) qgemm_wide_q6k_kernel<2><<<(unsigned)grid, WT, 0, ctx->stream>>>(a);
-        else if (q6k) qgemm_wide_q6k_kernel<4><<<(unsigned)grid, WT, 0, ctx->stream>>>(a);
-        else if (a.M <= 16) qgemm_wide_kernel<1><<<(unsigned)grid, WT, 0, ctx->stream>>>(a);
-        else if (a.M <= 32) qgemm_wide_kernel<2><<<(unsigned)grid, WT, 0, ctx->stream>>>(a);
-        else qgemm_wide_kernel<4><<<(unsigned)grid, WT, 0, ctx->stream>>>(a);
+        else if (q6k) kq_launch<CPV_Q6_K>(a, nmt, (unsigned)grid, ctx->stream);
+        else kq_launch<CPV_Q4_K>(a, nmt, (unsigned)grid, ctx->stream);
+        if (y && rest)
+            wide_finalize_kernel<<<dim3((unsigned)rest, (unsigned)nmt), WT, 0, ctx->stream>>>(
+                a, a.U * (q80 ? 8 : 1), nmt * 16);
     };
     go();
     CPV_HIP(ctx, hipGetLastError());

@@ -111,6 +111,26 @@ def test_qgemm_wide_bit_exact_small(ctx, tname, n, k, m):
     assert np.array_equal(y.view(np.uint32), ref.view(np.uint32)), np.abs(y - ref).max()
 
 
+@pytest.mark.parametrize("tname", ["q4_k", "q6_k", "q8_0"])
+@pytest.mark.parametrize("m", [9, 16, 17, 33, 49, 65, 81, 97, 113, 128, 129, 145, 255])
+def test_qgemm_wide_row_blocks(ctx, tname, m):
+    # every number of 16-row blocks a workgroup holds, with one row in the last
+    # block or all; weight rows past a tile; 11 units, which no slice count divides
+    y, ref = run_case(ctx, TYPES[tname], 131, 2816, m)
+    assert np.array_equal(y.view(np.uint32), ref.view(np.uint32)), np.abs(y - ref).max()
+
+
+@pytest.mark.parametrize("tname", ["q4_k", "q6_k", "q8_0"])
+def test_qgemm_wide_whole_and_sliced(ctx, tname):
+    # more (tile, row block) pairs than workgroups in flight: whole rounds run
+    # over all of K, the rest in K slices through the accumulator; twice, as
+    # the accumulator has to be zero again
+    t, n, k, m = TYPES[tname], 64 * 810 + 3, 2048, 40
+    for seed in (0, 1):
+        y, ref = run_case(ctx, t, n, k, m, seed=seed)
+        assert np.array_equal(y.view(np.uint32), ref.view(np.uint32)), np.abs(y - ref).max()
+
+
 @pytest.mark.parametrize("m", [32, 100])
 def test_qgemm_wide_q8_0_partial_unit(ctx, m):
     # K = 800: 25 blocks of 32, so the last 256-element unit holds one block
