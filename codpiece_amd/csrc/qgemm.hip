@@ -1107,13 +1107,7 @@ static cpv_status qgemm_into(cpv_ctx* ctx, const cpv_weight* w, const cpv_act* a
                                      : lds_of<CPV_Q8_0>(M, a.nu_max, a.nt_max);
     };
     if (cpv_qgemm_wide_ok(w, m)) {
-        const bool own = w->type != CPV_Q8_0;   // (the K-quants' kernel writes y itself)
-        if ((st = cpv_qgemm_wide(ctx, w, act, a.gsum, a.win, own ? y : nullptr)) != CPV_OK) return st;
-        if (y && !own)
-            qgemm_finalize_kernel<<<dim3((unsigned)((w->n + 255) / 256), (unsigned)m), 256, 0, ctx->stream>>>(
-                a.gsum, a.n_pad, a.ew, a.da, 8 * U, 0, a.win, y, w->n);
-        CPV_HIP(ctx, hipGetLastError());
-        return CPV_OK;
+        return cpv_qgemm_wide(ctx, w, act, a.gsum, a.win, y);
     }
     const size_t lds_cap = ctx->lds_max - 1024;
     for (int64_t m0 = 0; m0 < m;) {

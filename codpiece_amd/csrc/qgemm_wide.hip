@@ -25,12 +25,12 @@
 
 namespace {
 
-constexpr int WBM = 64;                 // activation rows per workgroup
 constexpr int WT = 256;                 // threads per workgroup (4 waves)
-constexpr int WROW = 256 + 16;          // LDS bytes per staged activation row (+16 spreads the banks)
-constexpr int MAX_NMT = 8;              // 16-row activation blocks per workgroup (K-quants)
-// workgroups per CU: three waves per SIMD hold 168 registers, up to two blocks
-constexpr int wide_per_cu(int nmt) { return nmt > 2 ? 2 : 3; }
+constexpr int MAX_NMT = 8;              // 16-row activation blocks per workgroup, K-quants
+constexpr int MAX_NMT_Q80 = 4;          //   and Q8_0 (its scales' LDS at 4 lets three share a CU)
+// workgroups per CU: three waves per SIMD hold 168 registers (K-quants: up to
+// two blocks)
+constexpr int wide_per_cu(bool q80, int nmt) { return !q80 && nmt > 2 ? 2 : 3; }
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v2i __attribute__((ext_vector_type(2)));
@@ -52,6 +52,7 @@ struct WideArgs {
     const int32_t* bs16;   // [rows][U*16] sums of 16 codes (Q8_K)
     float* y;              // outputs [rows][n], or null: the sums stay in gsum
     int64_t n;             // weight rows
+    bool vec;              // y takes 16-byte stores (n a multiple of 4, y aligned)
     int nfull;             // (tile, row block) pairs that run over all of K
 };
 
@@ -64,6 +65,21 @@ __device__ __forceinline__ v4i mfma16(int64_t a, int64_t b, v4i c)
 {
     return __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b, c, 0, 0, 0);
 }
+
+// 16 bytes per lane from g into LDS at dst + 16 lane (dst wave-uniform), past
+// the registers.  Written out because the builtin makes the compiler wait for
+// the transfer before the next LDS read of any address (it cannot tell the two
+// buffers apart): the unit then stalled for its successor's loads (17408 x 5120
+// at 256 rows: 95 us a call, 90 this way).  The caller waits
+// (wide_dma_wait) before the barrier that publishes dst.  (The s_nop: a wait
+// state between the write of m0 and its use.)
+__device__ __forceinline__ void wide_dma16(const void* g, void* dst)
+{
+    const uint32_t l = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)dst;
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+                 : : "v"(g), "s"(__builtin_amdgcn_readfirstlane(l)) : "m0", "memory");
+}
+__device__ __forceinline__ void wide_dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 struct WidePart { int pair, u0, u1; bool whole; };
 
@@ -192,7 +208,7 @@ struct KqLds {
 };
 
 template <int TYPE, int NMT>
-__global__ __launch_bounds__(WT) __attribute__((amdgpu_waves_per_eu(wide_per_cu(NMT)))) void qgemm_wide_kq_kernel(WideArgs a)
+__global__ __launch_bounds__(WT) __attribute__((amdgpu_waves_per_eu(wide_per_cu(false, NMT)))) void qgemm_wide_kq_kernel(WideArgs a)
 {
     constexpr bool Q4 = TYPE == CPV_Q4_K;
     constexpr int R = 16 * NMT, PCS = Q4 ? 9 : 13;
@@ -226,9 +242,7 @@ __global__ __launch_bounds__(WT) __attribute__((amdgpu_waves_per_eu(wide_per_cu(
     auto stage_load = [&](int u, int buf, Stage& t) {
 #pragma unroll
         for (int q = 0; q < NMT; q++)
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(qbase + soff[q] + u * 256),
-                                             (__attribute__((address_space(3))) void*)&s.codes[buf][(q * 4 + wave) * 4][0],
-                                             16, 0, 0);
+            wide_dma16(qbase + soff[q] + u * 256, &s.codes[buf][(q * 4 + wave) * 4][0]);
         if constexpr (Q4) {
             t.b[0] = *(const v4i*)(sbs + u * 16);
             t.b[1] = *(const v4i*)(sbs + u * 16 + 4);
@@ -283,6 +297,7 @@ __global__ __launch_bounds__(WT) __attribute__((amdgpu_waves_per_eu(wide_per_cu(
     stage_load(u0, 0, st);
     __syncthreads();                     // s.sm
     stage_store(0, st);
+    wide_dma_wait();
     __syncthreads();
 
     for (int u = u0; u < u1; u++) {
@@ -417,91 +432,92 @@ __global__ __launch_bounds__(WT) __attribute__((amdgpu_waves_per_eu(wide_per_cu(
             __builtin_amdgcn_sched_barrier(0);
         }
         stage_store(buf ^ 1, st);
+        wide_dma_wait();
         __syncthreads();
         wc = wn;
     }
     wide_store<NMT>(a, wp, tile, rbase, nrow, g, er, s_ea, S);
 }
 
-// The same for Q8_0 weights and activations (ggml's Q8_0 vec_dot_type).
-// Per (activation row m, weight row n, 32-element block j) the dot is one
+// ---------------------------------------------------------------- Q8_0
+// The same for Q8_0 weights and activations (ggml's Q8_0 vec_dot_type).  Per
+// (activation row m, weight row n, 32-element block j) the dot is one
 // 16x16x32 MFMA's entry, and the block's term is rounded on its own:
-//     term = rint(dw_j * da_j * 2^-g * dot)          (binary64, exact product)
-// eight terms per 256-element unit where Q4_K has two, so this kernel is
-// bound by its binary64 VALU work.  A unit's 17 pieces: 16 of codes (block j
-// in pieces 2j, 2j + 1), then the 8 block scales (f16).
-// NMT: 16-row blocks of the 64 that hold rows (fewer when M <= 48)
+//     term = rint(dw_j * da_j * 2^-g * dot)          (binary64)
+// eight terms per 256-element unit, so VALU issue bounds this kernel: four
+// instructions a term.  The product is exact (11 + 11 + 20 bits), so one fma
+// with +-1.5 * 2^52 rounds it to its integer as rint does (|term| < 2^51);
+// the terms of blocks 2 p and 2 p + 1 carry opposite offsets, and their sum is
+// the two integers' (exact, and infinities and NaN pass as they did).  A lane
+// holds one activation row and 4 weight rows (the weights are the MFMA's A
+// operand): a block's activation scale is then one 8-byte LDS read per 4
+// terms, where 4 rows' scales were 4 reads and LDS the bound.  The two MFMAs
+// of the next block pair and row block run beside a pair's terms.
+// 7168 x 5120 at 201 rows, whole call: 121 -> 63 us; 17408 x 5120 at 256 rows: 226 -> 148.
+// A unit's 17 pieces: 16 of codes (block j in pieces 2j, 2j + 1), then the 8
+// block scales (f16).
 template <int NMT>
-__global__ __launch_bounds__(WT) __attribute__((amdgpu_waves_per_eu(2))) void qgemm_wide_q80_kernel(WideArgs a)
+__global__ __launch_bounds__(WT) __attribute__((amdgpu_waves_per_eu(3))) void qgemm_wide_q80_kernel(WideArgs a)
 {
-    __shared__ __align__(16) uint8_t s_codes[2][16 * NMT][WROW];
-    __shared__ double s_dad[2][16 * NMT + 1][8];   // da_j * 2^(win - Ea) per staged row and block (+ a dump row)
-    __shared__ double s_sm[WBM];         // 2^(win - Ea(m)), 0 for an all-zero row
+    constexpr int R = 16 * NMT, STEPS = 4 * NMT;
+    struct Lds {
+        uint8_t codes[2][R][256];        // 16-byte piece p of row r at slot p ^ (r % 16)
+        double dad[2][8][R];             // da_j * 2^(win - Ea) per block and staged row
+        double dw[2][8][64];             // dw_j * 2^-Ew per block and weight row
+        double sm[R];                    // 2^(win - Ea(m)), 0 for an all-zero row
+    };
+    __shared__ __align__(16) Lds s;
+    __shared__ int s_ea[R];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int U = a.U, M = a.M, NDA = 8 * a.U;
     const int64_t Kp = (int64_t)U * 256;
+    const WidePart wp = wide_part(a, blockIdx.x);
+    const int tile = wp.pair / a.mblocks, rbase = (wp.pair - tile * a.mblocks) * R, u0 = wp.u0, u1 = wp.u1;
 
-    const int nb = gridDim.x, b0 = blockIdx.x;
-    const int L = (nb & 7) == 0 ? (b0 & 7) * (nb >> 3) + (b0 >> 3) : b0;
-    const int mb = L % a.mblocks, r0 = L / a.mblocks;
-    const int ks = r0 % a.ksplit, tile = r0 / a.ksplit;
-    const int u0 = ks * a.upk, u1 = min(U, u0 + a.upk);
-    const int rbase = mb * WBM;
+    wide_row_exponents<NMT>(a, rbase, NDA, s.sm, s_ea);
 
-    for (int r = wave; r < WBM; r += WT / 64) {
-        const int mr = a.m0 + min(rbase + r, M - 1);
-        float mx = 0.0f;
-        for (int c = lane; c < NDA; c += 64) mx = fmaxf(mx, fabsf(a.da[(int64_t)mr * NDA + c]));
-        mx = cpv_wave_reduce(mx, cpv_op_max());
-        if (lane == 0) {
-            int e = CPV_E_EMPTY;
-            if (mx > 0.0f) frexpf(mx, &e);
-            s_sm[r] = e == CPV_E_EMPTY ? 0.0 : ldexp(1.0, a.win - e);
-        }
-    }
-
-    const int8_t* qbase = a.qa + (int64_t)(a.m0 + rbase) * Kp;
-    int soff[4];
+    // staging of one unit: the codes from memory into LDS directly (as the
+    // K-quants'); the scales of two blocks per thread, of the activations (8 R
+    // / 2 threads, the others repeat them) and of the weights
+    const int8_t* qbase = a.qa + (int64_t)rbase * Kp;
+    int soff[NMT];
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const int p = tid + q * WT, r = p >> 4;
-        soff[q] = (min(rbase + r, M - 1) - rbase) * (int)Kp + (p & 15) * 16;
+    for (int q = 0; q < NMT; q++) {
+        const int r = (q * 4 + wave) * 4 + (lane >> 4);
+        soff[q] = (min(rbase + r, M - 1) - rbase) * (int)Kp + ((lane & 15) ^ (r & 15)) * 16;
     }
-    // scales: thread tid stages blocks 2 (tid & 3), +1 of row tid >> 2
-    const int srow = tid >> 2, sblk = 2 * (tid & 3);
-    const float* sda = a.da + (int64_t)(a.m0 + min(rbase + srow, M - 1)) * NDA + sblk;
-    auto stage_load = [&](int u, v4i* cv, float2& dv) {
+    const int arow = (tid >> 2) % R, ablk = 2 * (tid & 3), wsrow = tid & 63, wsblk = 2 * (tid >> 6);
+    const float* sda = a.da + (int64_t)min(rbase + arow, M - 1) * NDA + ablk;
+    const uint8_t* wtile = a.w + (int64_t)tile * U * 17 * 1024;
+    const int ews = a.ew[(int64_t)tile * 64 + wsrow];
+    struct Stage { float2 d; uint32_t w; };
+    auto stage_load = [&](int u, int buf, Stage& t) {
 #pragma unroll
-        for (int q = 0; q < NMT; q++) cv[q] = *(const v4i*)(qbase + soff[q] + u * 256);
-        dv = *(const float2*)(sda + 8 * u);
+        for (int q = 0; q < NMT; q++)
+            wide_dma16(qbase + soff[q] + u * 256, &s.codes[buf][(q * 4 + wave) * 4][0]);
+        t.d = *(const float2*)(sda + 8 * u);
+        t.w = *(const uint32_t*)(wtile + ((int64_t)u * 17 + 16) * 1024 + wsrow * 16 + wsblk * 2);
     };
-    auto stage_store = [&](int buf, const v4i* cv, float2 dv) {
-#pragma unroll
-        for (int q = 0; q < NMT; q++) {
-            const int p = tid + q * WT;
-            *(v4i*)&s_codes[buf][p >> 4][(p & 15) * 16] = cv[q];
-        }
-        // (rows past the blocks write the dump row: a branch here made the
-        // compiler hold every load across it, 256 VGPRs and spills)
-        const int sr = srow < 16 * NMT ? srow : 16 * NMT;
-        s_dad[buf][sr][sblk] = (double)dv.x * s_sm[srow];
-        s_dad[buf][sr][sblk + 1] = (double)dv.y * s_sm[srow];
+    auto stage_store = [&](int buf, const Stage& t) {
+        s.dad[buf][ablk][arow] = (double)t.d.x * s.sm[arow];
+        s.dad[buf][ablk + 1][arow] = (double)t.d.y * s.sm[arow];
+        s.dw[buf][wsblk][wsrow] = ldexp((double)cpv_h2f((uint16_t)(t.w & 0xffffu)), -ews);
+        s.dw[buf][wsblk + 1][wsrow] = ldexp((double)cpv_h2f((uint16_t)(t.w >> 16)), -ews);
     };
 
-    // this lane's weight row and k slot: 8 codes of block j (bytes 8 (kq & 1)
-    // .. of piece 2j + (kq >> 1)), and the row's 8 block scales
-    const int nl = lane & 15, kq = lane >> 4;
-    const int nrow = wave * 16 + nl;
-    const uint8_t* wrow = a.w + (int64_t)tile * U * 17 * 1024 + nrow * 16;
-    struct Wt { v2i q[8]; v4i s; };
+    // this lane's weight row and k slot: 8 codes of block j (bytes 8 (g & 1)
+    // .. of piece 2j + (g >> 1))
+    const int nl = lane & 15, g = lane >> 4;
+    const uint8_t* wrow = wtile + (wave * 16 + nl) * 16 + (g >> 1) * 1024 + 8 * (g & 1);
+    struct Wt { v2i q[8]; };
     auto wload = [&](int u, Wt& t) {
-        const uint8_t* p = wrow + (int64_t)u * 17 * 1024;
 #pragma unroll
-        for (int j = 0; j < 8; j++) t.q[j] = *(const v2i*)(p + (2 * j + (kq >> 1)) * 1024 + 8 * (kq & 1));
-        t.s = *(const v4i*)(p + 16 * 1024);
+        for (int j = 0; j < 8; j++) t.q[j] = *(const v2i*)(wrow + ((int64_t)u * 17 + 2 * j) * 1024);
     };
-    const int er = a.ew[(int64_t)tile * 64 + nrow];
+    // the lane's outputs: weight rows n0 .. n0 + 3
+    const int64_t n0 = (int64_t)tile * 64 + wave * 16 + 4 * g;
+    const double MAGIC = 0x1.8p52;
 
     double S[NMT][4];
 #pragma unroll
@@ -510,51 +526,127 @@ __global__ __launch_bounds__(WT) __attribute__((amdgpu_waves_per_eu(2))) void qg
         for (int i = 0; i < 4; i++) S[mt][i] = 0.0;
 
     Wt wc, wn;
-    v4i cv[NMT];
-    float2 dv;
+    Stage st;
     wload(u0, wc);
-    stage_load(u0, cv, dv);
-    __syncthreads();                    // s_sm
-    stage_store(0, cv, dv);
+    stage_load(u0, 0, st);
+    __syncthreads();                     // s.sm
+    stage_store(0, st);
+    wide_dma_wait();
     __syncthreads();
 
     for (int u = u0; u < u1; u++) {
         const int buf = (u - u0) & 1;
-        const int un = u + 1 < u1 ? u + 1 : u;
+        const int un = u + 1 < u1 ? u + 1 : u;   // (the last one reloads itself: no branch)
         wload(un, wn);
-        stage_load(un, cv, dv);
+        stage_load(un, buf ^ 1, st);
+        const uint8_t* cb = &s.codes[buf][0][0] + nl * 256 + 8 * (g & 1);
+        // step t: block pair p = t / NMT, row block t % NMT
+        int64_t av[2];
+        double da[2], dan[2], dw[2][4];
+        auto fetch = [&](int t) {
+            const int p = t / NMT, mt = t % NMT;
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const uint32_t hw = (uint32_t)wc.s[j >> 1];
-            const double dwj = ldexp((double)cpv_h2f((uint16_t)((j & 1) ? hw >> 16 : hw & 0xffffu)), -er);
-            const int64_t bq = pack2((uint32_t)wc.q[j][0], (uint32_t)wc.q[j][1]);
+            for (int h = 0; h < 2; h++)
+                av[h] = *(const int64_t*)(cb + mt * 4096 + ((2 * (2 * p + h) + (g >> 1)) ^ nl) * 16);
+        };
+        auto fetch_d = [&](int t) {
+            const int p = t / NMT, mt = t % NMT;
 #pragma unroll
-            for (int mt = 0; mt < NMT; mt++) {
-                const int64_t av = *(const int64_t*)&s_codes[buf][mt * 16 + nl][8 * kq + 32 * j];
-                const v4i d = mfma16(av, bq, v4i{0, 0, 0, 0});
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-                    S[mt][i] += rint(dwj * s_dad[buf][mt * 16 + 4 * kq + i][j] * (double)d[i]);   // |dot| <= 32*127*127
+            for (int h = 0; h < 2; h++) {
+                dan[h] = s.dad[buf][2 * p + h][mt * 16 + nl];
             }
+        };
+        auto fetch_w = [&](int p) {
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) dw[h][i] = s.dw[buf][2 * p + h][wave * 16 + 4 * g + i];
+        };
+        struct Acc { v4i d[2]; };
+        auto mma = [&](int t, Acc& c) {
+            const int p = t / NMT;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int j = 2 * p + h;
+                c.d[h] = mfma16(pack2((uint32_t)wc.q[j][0], (uint32_t)wc.q[j][1]), av[h], v4i{0, 0, 0, 0});
+            }
+        };
+        Acc c[2];
+        fetch(0);
+        fetch_d(0);
+        fetch_w(0);
+        mma(0, c[0]);
+        fetch(1 < STEPS ? 1 : 0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = 0; t < STEPS; t++) {
+            const int mt = t % NMT;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                da[h] = dan[h];
+            }
+            if (t + 1 < STEPS) {
+                mma(t + 1, c[(t + 1) & 1]);
+                if (t + 2 < STEPS) fetch(t + 2);
+                fetch_d(t + 1);
+            }
+            const Acc& x = c[t & 1];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const double ta = __builtin_fma(dw[0][i] * da[0], (double)x.d[0][i], MAGIC);
+                const double tb = __builtin_fma(dw[1][i] * da[1], (double)x.d[1][i], -MAGIC);
+                S[mt][i] += ta + tb;
+            }
+            if (mt == NMT - 1 && t + 1 < STEPS) fetch_w((t + 1) / NMT);
             __builtin_amdgcn_sched_barrier(0);
         }
-        stage_store(buf ^ 1, cv, dv);
+        stage_store(buf ^ 1, st);
+        wide_dma_wait();
         __syncthreads();
         wc = wn;
     }
 
-    double* g = a.gsum + (int64_t)tile * 64 + nrow;
+    // the outputs directly, or the sums to the accumulator: from a transposed
+    // copy in LDS, so that 16 lanes' adds are 16 weight rows of one activation
+    // row (adds scattered over rows took twice the whole launch)
+    if (a.y && wp.whole) {
+        int er[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) er[i] = a.ew[n0 + i];
+#pragma unroll
+        for (int mt = 0; mt < NMT; mt++) {
+            const int m = rbase + mt * 16 + nl;
+            if (m >= M) continue;
+            float* y = a.y + (int64_t)m * a.n + n0;
+            float v[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) v[i] = cpv_gout_value(S[mt][i], er[i], s_ea[mt * 16 + nl], a.win);
+            if (a.vec) {   // (n a multiple of 4, y 16-byte aligned: the four rows exist together)
+                if (n0 < a.n) *(float4*)y = float4{v[0], v[1], v[2], v[3]};
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (n0 + i < a.n) y[i] = v[i];
+            }
+        }
+        return;
+    }
+    static_assert(sizeof(s.codes) >= 64 * R * sizeof(double), "the sums fit the staged codes' space");
+    double* sS = (double*)&s.codes[0][0][0] + wave * 16 * R;   // (the loop's last barrier is past: the codes are read)
 #pragma unroll
     for (int mt = 0; mt < NMT; mt++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int m = rbase + mt * 16 + 4 * kq + i;
-            if (m < M) {
-                double* p = g + (int64_t)(a.m0 + m) * a.n_pad;
-                if (a.ksplit == 1) *p = S[mt][i];
-                else unsafeAtomicAdd(p, S[mt][i]);
-            }
-        }
+        for (int i = 0; i < 4; i++) sS[(mt * 16 + nl) * 16 + 4 * g + i] = S[mt][i];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4 * NMT; q++) {
+        const int r = 4 * q + g, m = rbase + r;
+        if (m >= M) continue;
+        const double v = sS[r * 16 + nl];
+        double* p = a.gsum + (int64_t)m * a.n_pad + (int64_t)tile * 64 + wave * 16 + nl;
+        if (wp.whole) *p = v;
+        else unsafeAtomicAdd(p, v);
+    }
 }
 
 }  // namespace
@@ -573,31 +665,33 @@ namespace {
 // Rows per workgroup and the deal of the (tile, row block) pairs over the
 // chip's slots (workgroups in flight).  Whole rounds of pairs run over all of
 // K; the pairs that are left run in ks K slices of at least 4 units each.
-// Chosen by an estimate in us, from gate|up (17408 and 34816 x 5120), wo and
-// down (5120 x 5120, 5120 x 17408) at 128 to 256 rows: a unit takes 0.7 +
-// 0.335 nmt with the CU full and 0.62 of that with one workgroup on it, a
-// workgroup's start (row exponents, first loads) 3, and a million atomic adds
-// of a slice's sums 3.5 (they bypass the XCD's L2).  E.g. 17408 x 5120 at 128
-// rows: 8 blocks in 272 pairs 76 us a call, 4 in 544 pairs 62; 5120 x 17408 at
-// 256 rows: 8 blocks in 160 pairs x 3 slices 116, 4 in 320 whole pairs 146.
-void wide_split(WideArgs& a, int cus, int* nmt_out)
+// Chosen by an estimate in us, from 5120, 7168, 12288, 17408 and 34816 x 5120
+// and 5120 x 17408 at 64 to 256 rows: a unit of nmt row blocks takes 0.5 +
+// 0.315 nmt with two workgroups on a CU (Q8_0: 0.95 nmt with three) and 0.62
+// of that with one, a workgroup's start (row exponents, first loads) 3, and a
+// million atomic adds of a slice's sums 3.5 (they bypass the XCD's L2).  E.g.
+// Q4_K 17408 x 5120 at 128 rows: 8 blocks in 272 pairs 70 us a call, 4 in 544
+// pairs 55; 5120 x 17408 at 256 rows: 8 blocks in 160 pairs x 3 slices 112, 4
+// in 320 whole pairs 146; Q8_0 7168 x 5120 at 201 rows: 3 blocks in 560 pairs
+// 75, 2 in 784 pairs 63.
+void wide_split(WideArgs& a, bool q80, int cus, int* nmt_out)
 {
     const int nb16 = (a.M + 15) / 16;
     double best = 1e30;
-    for (int mb = (nb16 + MAX_NMT - 1) / MAX_NMT; mb <= nb16; mb++) {
+    const int maxb = q80 ? MAX_NMT_Q80 : MAX_NMT;
+    for (int mb = (nb16 + maxb - 1) / maxb; mb <= nb16; mb++) {
         const int nmt = (nb16 + mb - 1) / mb;
         if ((nb16 + nmt - 1) / nmt != mb) continue;   // (the same blocks in fewer workgroups)
-        const int slots = cus * wide_per_cu(nmt);
+        const int slots = cus * wide_per_cu(q80, nmt);
         const int64_t pairs = (int64_t)a.tiles * mb, full = pairs / slots * slots, rest = pairs - full;
-        const double t = (0.7 + 0.335 * nmt) * wide_per_cu(nmt) / 2, t1 = 0.62 * t, s0 = 3.0;
+        const double t = q80 ? 0.95 * nmt : (0.5 + 0.315 * nmt) * wide_per_cu(q80, nmt) / 2, t1 = 0.62 * t, s0 = 3.0;
         const double tf = (double)(full / slots) * (a.U * t + s0);
         for (int ks = 1; ks == 1 || (rest && ks <= a.U / 4 && ks <= 16); ks++) {
             const int upk = (a.U + ks - 1) / ks, k2 = (a.U + upk - 1) / upk;
             if (k2 != ks) continue;
             const int64_t w = rest * ks, last = w % slots;
             double tr = (double)(w / slots) * (upk * t + s0);
-            // (one workgroup a CU up to cus, then a share of the CUs full)
-            if (last) tr += upk * (last > cus ? t1 + (t - t1) * (double)(last - cus) / (slots - cus) : t1) + s0;
+            if (last) tr += upk * (last > cus ? t : t1) + s0;   // (past cus the fullest CU decides)
             if (ks > 1) tr += (double)w * nmt * 1024 * 3.5e-6 + 1.5;
             if (tf + tr < best) {
                 best = tf + tr;
@@ -609,6 +703,16 @@ void wide_split(WideArgs& a, int cus, int* nmt_out)
             }
         }
         if (nmt <= 2) break;
+    }
+}
+
+void q80_launch(const WideArgs& a, int nmt, unsigned grid, hipStream_t stream)
+{
+    switch (nmt) {
+    case 1: qgemm_wide_q80_kernel<1><<<grid, WT, 0, stream>>>(a); break;
+    case 2: qgemm_wide_q80_kernel<2><<<grid, WT, 0, stream>>>(a); break;
+    case 3: qgemm_wide_q80_kernel<3><<<grid, WT, 0, stream>>>(a); break;
+    default: qgemm_wide_q80_kernel<4><<<grid, WT, 0, stream>>>(a); break;
     }
 }
 
@@ -635,7 +739,7 @@ cpv_status cpv_qgemm_wide(cpv_ctx* ctx, const cpv_weight* w, const cpv_act* act,
     if ((w->type != CPV_Q4_K && !q80 && !q6k) || act->kq == q80 || act->U != (int)w->units || act->m < 1 ||
         act->m > INT32_MAX / 2)
         return cpv_fail(ctx, CPV_EINVAL, "qgemm_wide: weight or activation format not supported");
-    if (2LL * WBM * act->U * 256 > INT32_MAX)   // the staging offsets within a row block are 32-bit
+    if (16LL * MAX_NMT * act->U * 256 > INT32_MAX)   // the staging offsets within a row block are 32-bit
         return cpv_fail(ctx, CPV_EUNSUPPORTED, "qgemm_wide: k=%lld too long", (long long)w->k);
     WideArgs a;
     a.w = (const uint8_t*)w->data;
@@ -652,28 +756,16 @@ cpv_status cpv_qgemm_wide(cpv_ctx* ctx, const cpv_weight* w, const cpv_act* act,
     a.bs16 = act->bs16;
     a.y = y;
     a.n = w->n;
+    a.vec = (w->n & 3) == 0 && ((uintptr_t)y & 15) == 0;
     if ((int64_t)a.tiles * ((a.M + 15) / 16) > INT32_MAX / 1024)
         return cpv_fail(ctx, CPV_EUNSUPPORTED, "qgemm_wide: %d tiles by %d rows", a.tiles, a.M);
     int nmt = 4;
-    if (q80) {
-        // slice K when the grid would leave CUs idle (about 3 workgroups fit a CU)
-        a.mblocks = (a.M + WBM - 1) / WBM;
-        const int64_t blocks = (int64_t)a.tiles * a.mblocks, want = 3LL * ctx->cu_count;
-        int ksplit = blocks >= want ? 1 : (int)((want + blocks - 1) / blocks);
-        if (ksplit > a.U / 4) ksplit = a.U / 4 > 1 ? a.U / 4 : 1;
-        a.upk = (a.U + ksplit - 1) / ksplit;
-        a.ksplit = (a.U + a.upk - 1) / a.upk;
-        a.nfull = 0;
-    } else {
-        wide_split(a, ctx->cu_count, &nmt);
-    }
+    wide_split(a, q80, ctx->cu_count, &nmt);
     const int64_t blocks = (int64_t)a.tiles * a.mblocks;
     const int64_t rest = blocks - a.nfull, grid = a.nfull + rest * a.ksplit;
     const int ev = cpv_prof_mark(ctx);
     auto go = [=]() {
-        if (q80 && a.M <= 16) qgemm_wide_q80_kernel<1><<<(unsigned)grid, WT, 0, ctx->stream>>>(a);
-        else if (q80 && a.M <= 32) qgemm_wide_q80_kernel<2><<<(unsigned)grid, WT, 0, ctx->stream>>>(a);
-        else if (q80) qgemm_wide_q80_kernel<4><<<(unsigned)grid, WT, 0, ctx->stream>>>(a);
+        if (q80) q80_launch(a, nmt, (unsigned)grid, ctx->stream);
         else if (q6k) kq_launch<CPV_Q6_K>(a, nmt, (unsigned)grid, ctx->stream);
         else kq_launch<CPV_Q4_K>(a, nmt, (unsigned)grid, ctx->stream);
         if (y && rest)
