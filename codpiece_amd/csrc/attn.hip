@@ -51,6 +51,8 @@ constexpr int VLIMBS = CPV_ATTN_VLIMBS;
 constexpr int QB_CHAIN = 32;        // query rows per chunk workgroup: chains, prefill, fewer than 512 units;
 constexpr int QB_WIDE = 48;         //   from 512 (chunk, KV head) units on, when a KV head has more than 32,
 constexpr int QB_TREE = 80;         //   or, over the API's caches, 49 to 80 (a 16-node tree's 5 x 16)
+constexpr int64_t LIMB_ROWS = 512;  // query rows per KV head from which the API's caches become limb caches first
+constexpr size_t LIMB_BYTES = (size_t)256 << 20;   //   and the most those may take
 constexpr int E_EMPTY = CPV_E_EMPTY;   // exponent of an all-zero vector
 
 __device__ __forceinline__ int ceil_log2_dev(int64_t v)
@@ -178,6 +180,62 @@ __global__ __launch_bounds__(256) void q_limbs_kernel(const float* __restrict__ 
         *(uint4*)(dst + D) = uint4{lo[0], lo[1], lo[2], lo[3]};
         if (sub == 0) qexp[row] = e;
     }
+}
+
+// The API's f16 caches as a session's limb caches (the layouts the LC kernels
+// read), once per call (attn_run).  4096 rows of 8 heads x 128: 11.6 us for 16
+// MB in and 25 MB out.  K: TPR lanes per row and head, as the chunk
+// kernel converts it; V: a thread takes 16 rows of one column.
+template <int D>
+__global__ __launch_bounds__(256) void kv_limbs_kernel(const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vt,
+                                                       int64_t v_stride, int64_t n, int64_t ls, int Hkv,
+                                                       int8_t* __restrict__ kl, int8_t* __restrict__ vl, int k_blocks)
+{
+    constexpr int TPR = D / 16;
+    if ((int)blockIdx.x < k_blocks) {          // (whole workgroups)
+        const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x, rh = g / TPR, rows = n * Hkv;
+        const int sub = (int)(g % TPR);
+        const int64_t rc = rh < rows ? rh : rows - 1;   // (a row's lanes reduce together: all active)
+        const uint4* src = (const uint4*)(kc + rc * D + sub * 16);
+        const uint4 x0 = src[0], x1 = src[1];
+        const uint32_t wds[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+        float v[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) v[i] = cpv_h2f((uint16_t)(wds[i >> 1] >> (16 * (i & 1))));
+        uint32_t hi[4], lo[4];
+        const int e = row_limbs<TPR>(v, hi, lo);
+        if (rh >= rows) return;
+        const int64_t row = rc / Hkv;
+        const int kh = (int)(rc - row * Hkv);
+        int8_t* dst = kl + row * cpv_k_row_bytes(Hkv, D) + (int64_t)kh * 2 * D + sub * 16;
+        *(uint4*)dst = uint4{hi[0], hi[1], hi[2], hi[3]};
+        *(uint4*)(dst + D) = uint4{lo[0], lo[1], lo[2], lo[3]};
+        if (sub == 0) cpv_k_exps((int32_t*)kl, Hkv, D, ls)[(int64_t)kh * ls + row] = e;
+        return;
+    }
+    const int64_t g = (int64_t)(blockIdx.x - k_blocks) * 256 + threadIdx.x, segs = ls / 16;
+    const int64_t col = g / segs, seg = g - col * segs;
+    if (col >= (int64_t)Hkv * D) return;
+    // (rows past the cache's stride, in the last segment, as zeros; those past n carry weight 0)
+    const uint16_t* src = vt + col * v_stride + seg * 16;
+    const uint4 x0 = seg * 16 < v_stride ? *(const uint4*)src : uint4{0, 0, 0, 0};
+    const uint4 x1 = seg * 16 + 8 < v_stride ? *(const uint4*)(src + 8) : uint4{0, 0, 0, 0};
+    const uint32_t wds[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+    uint32_t pk[VLIMBS][4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        uint32_t w[4], t[VLIMBS];
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            w[k] = packed_limbs<VLIMBS>(
+                (int)rintf(ldexpf(cpv_h2f((uint16_t)(wds[2 * j + (k >> 1)] >> (16 * (k & 1)))), VBITS)));
+        limb_transpose<VLIMBS>(w, t);
+#pragma unroll
+        for (int p = 0; p < VLIMBS; p++) pk[p][j] = t[p];
+    }
+    int8_t* dst = vl + (col * ls + seg * 16) * VLIMBS;
+#pragma unroll
+    for (int p = 0; p < VLIMBS; p++) *(uint4*)(dst + 16 * p) = uint4{pk[p][0], pk[p][1], pk[p][2], pk[p][3]};
 }
 
 // one 128-row chunk of the cache against QB query rows of one KV head
@@ -668,7 +726,7 @@ cpv_status attn_block(cpv_ctx* ctx, const float* q, const uint16_t* kc, const ui
                       int64_t n_past, const int32_t* parent, int T, int H, int Hkv, float scale, float* out,
                       cpv_attn_part* part = nullptr, const int64_t* pos = nullptr, int pos_sel = 0,
                       int nchunk_grid = 0, int64_t kv_rows = 0, const int8_t* vl = nullptr,
-                      const int8_t* kl = nullptr)
+                      const int8_t* kl = nullptr, size_t ws_off = 0)
 {
     if ((vl != nullptr) != (kl != nullptr))
         return cpv_fail(ctx, CPV_EINVAL, "attention: a session's K and V limb caches go together");
@@ -683,8 +741,9 @@ cpv_status attn_block(cpv_ctx* ctx, const float* q, const uint16_t* kc, const ui
     const size_t z_b = ((size_t)nchunk * rows * 8 + 255) & ~(size_t)255;
     const size_t ql_b = vl ? 0 : (((size_t)rows * 2 * D + 255) & ~(size_t)255) + (size_t)rows * 4;
     void* ws = nullptr;
-    cpv_status st = cpv_workspace(ctx, P_b + m_b + z_b + ql_b, &ws);
+    cpv_status st = cpv_workspace(ctx, ws_off + P_b + m_b + z_b + ql_b, &ws);
     if (st != CPV_OK) return st;
+    ws = (uint8_t*)ws + ws_off;                // (what lies before it is the caller's: attn_run's limb caches)
     ChunkArgs ca;
     ca.q = q;
     ca.qlim = nullptr;
@@ -785,10 +844,35 @@ cpv_status attn_run(cpv_ctx* ctx, const float* q, const uint16_t* kc, const uint
     int64_t tb = ((int64_t)192 << 20) / (per_token + 1);
     if (tb < 1) tb = 1;
     if (tb > t) tb = t;
+    // The API's caches under many query rows: made into limb caches first.
+    // Each block of 32 rows else converts every chunk's K and V again; from
+    // 512 rows per KV head the conversion's launch and the limbs' 1.5 times
+    // the bytes cost less (40/8 x 128, 3584 rows before: 640 rows 120 -> 113
+    // us, 2560 rows 480 -> 430; 320 rows 67.9 -> 67.8, and over 16384 rows
+    // 226 -> 252).
+    const int64_t ls = (n + 15) & ~(int64_t)15;
+    const size_t kl_b = ((size_t)cpv_k_cache_bytes(h_kv, D, ls) + 255) & ~(size_t)255;
+    const size_t vl_b = (size_t)h_kv * D * ls * VLIMBS;
+    size_t off = 0;
+    if (!vl && (int64_t)(h / h_kv) * t >= LIMB_ROWS && kl_b + vl_b <= LIMB_BYTES) {
+        // all of the call's workspace at once: growth would drop the caches
+        const int64_t rows = tb * h, nc = (n + CHUNK - 1) / CHUNK;
+        void* ws = nullptr;
+        cpv_status st = cpv_workspace(ctx, kl_b + vl_b + (size_t)nc * rows * (D * 4 + 12) + 3 * 256, &ws);
+        if (st != CPV_OK) return st;
+        const int64_t kb = (n * h_kv * (D / 16) + 255) / 256, vb = ((int64_t)h_kv * D * (ls / 16) + 255) / 256;
+        kv_limbs_kernel<D><<<(unsigned)(kb + vb), 256, 0, ctx->stream>>>(kc, vt, v_stride, n, ls, h_kv, (int8_t*)ws,
+                                                                        (int8_t*)ws + kl_b, (int)kb);
+        CPV_HIP(ctx, hipGetLastError());
+        kl = (int8_t*)ws;
+        vl = (int8_t*)ws + kl_b;
+        v_stride = ls;
+        off = kl_b + vl_b;
+    }
     for (int t0 = 0; t0 < t; t0 += (int)tb) {
         const int tn = t - t0 < (int)tb ? t - t0 : (int)tb;
         cpv_status st = attn_block<D>(ctx, q + (int64_t)t0 * h * D, kc, vt, v_stride, n_past + t0, nullptr, tn, h,
-                                      h_kv, scale, out + (int64_t)t0 * h * D, nullptr, nullptr, 0, 0, 0, vl, kl);
+                                      h_kv, scale, out + (int64_t)t0 * h * D, nullptr, nullptr, 0, 0, 0, vl, kl, off);
         if (st != CPV_OK) return st;
     }
     return CPV_OK;

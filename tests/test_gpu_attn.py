@@ -66,6 +66,15 @@ def test_27b_class_chain(ctx, n_past):
     close(*run(ctx, 5, 40, 8, 128, n_past, None))
 
 
+@pytest.mark.parametrize("t,h,hkv,d,n_past", [(128, 8, 2, 128, 0), (129, 16, 4, 64, 67), (256, 4, 2, 64, 401),
+                                              (103, 10, 2, 128, 1001)])
+def test_many_rows_take_limb_caches(ctx, t, h, hkv, d, n_past):
+    # 512 and more query rows per KV head: the caches are made into limbs
+    # first; n = 128, 196, 657, 1104 rows (strides that are and are not whole
+    # 16-row segments), and 515 rows, a last block of 3
+    close(*run(ctx, t, h, hkv, d, n_past, None, extra_rows=3))
+
+
 @pytest.mark.parametrize("n_ctx", [8192, 32768])
 def test_tree_verify_config(ctx, n_ctx):
     # 40 Q / 8 KV heads x 128, a 16-node draft tree over n_ctx context rows
