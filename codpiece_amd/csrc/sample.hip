@@ -650,6 +650,9 @@ __device__ __forceinline__ void sort_emit(const float* lg, int cnt, int pos, int
 // the split top-p build's state per row: the row maximum in EXP_SPLIT
 // parts, then what its first launch leaves for the second
 constexpr int EXP_SPLIT = 32;
+constexpr int FCAP = BAND / EXP_SPLIT;   // keys a part may select for a top-k or min-p build
+constexpr int FRONT_K = 256;             // top-k counts up to this select by parts
+constexpr int FT = 512;                  // threads of the part kernels (four workgroups share a CU)
 struct DistState {
     float sum1;                 // the index-order sum of exp(l - max)
     int cnt;                    // size of the first band
@@ -662,6 +665,11 @@ struct DistState {
     int boff[MAXP], bcnt[MAXP]; // each part's offset in the band and size
     unsigned long long first;   // the band's first key
     float bf1[MAXP], bf2[MAXP]; // each part's estimated sums of exp(l - max) and exp((l - max) / T)
+    // top-k and min-p builds (front_kernel, floor_kernel): each part's number
+    // of selected keys (kept in bkeys, FCAP a part), and the histogram bin
+    // they reach (top-k) or the number of logits at or above the floor (min-p)
+    int fcnt[EXP_SPLIT], fval[EXP_SPLIT];
+    int wn;                     // penalties: the window's distinct tokens (window_kernel)
     FMap m1[MAXP], m2[MAXP];    // each part's top-p fold (pr / sum1) and final-sum (exp(l / T - mx2)) steps
     int eb1[MAXP], eb2[MAXP];   // composed in these binades
 };
@@ -785,7 +793,7 @@ __device__ __noinline__ int emit_band(const float* lg, int V, bool have_last, un
 // histogram over the band's key range, each sorted by band_part_kernel).  Returns the band size and sets *last to its
 // last key and *np to the number of parts; or -1 (np = 0) when a part would
 // exceed SMALL_BAND keys, for the caller to emit the band itself.
-__device__ __noinline__ int emit_band_parts(const float* lg, int V, float mx, float T, unsigned long long* last,
+__device__ int emit_band_parts(const float* lg, int V, float mx, float T, unsigned long long* last,
                                             unsigned long long* bkeys, DistState* st, int* np,
                                             unsigned long long* keys, Small* sm)
 {
@@ -907,77 +915,93 @@ struct DistArgs {
     float* sl;                  // [rows][V] their (penalised, untempered) logits
     float* pr;                  // [rows][V] their probabilities
     int32_t* hdr;               // [rows] candidate count
-    int phase;                  // 0: the whole build; top-p split: 1 (two workgroups per row), then 2
     int pre_exp;                // top-p: pr already holds expf(l - max) (exp_kernel)
     DistState* st;              // [rows] (phases 1 and 2)
     unsigned long long* bkeys;  // [rows][BAND] the first band's keys, part by part (phase 1)
     float* e2;                  // [rows][BAND] exp(l / T - mx2) of the first band's candidates (band parts)
+    int sel;                    // the candidates come from front_kernel (top-k: the count) or floor_kernel (min-p: -1)
     int parts;                  // phase 1 leaves the first band in parts (band_part_kernel follows)
 };
 
-// Penalties (lib.rs:233-266): a dense copy of the row in which every token
-// of the window carries its penalised logit.  The window is the last
-// penalty_last_n of the history (valid entries, oldest first) followed by
-// the row's preceding drafts (Sampler::accept after each kept draft,
-// engine.rs:2368-2369).
-__device__ const float* apply_penalties(const float* logits, float* pen, int V, const int32_t* hist, int hist_len,
-                                        const int32_t* drafts, int nd, const cpv_sampler_params& P, int* win,
-                                        Small* sm)
+// Penalties (lib.rs:233-266): every token of the window carries its penalised
+// logit.  The window is the last penalty_last_n of the history (valid entries,
+// oldest first) followed by the row's preceding drafts (Sampler::accept after
+// each kept draft, engine.rs:2368-2369).  Per row, once: its distinct tokens
+// of the vocabulary with their counts (in e2's space, free until the band
+// parts), which front_kernel's parts apply.
+__global__ __launch_bounds__(FT) void window_kernel(DistArgs a)
 {
-    const int tid = threadIdx.x;
-    int valid[4], c = 0;
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const int a = tid * 4 + q;
-        valid[q] = (hist && a < hist_len && hist[a] >= 0) ? 1 : 0;
-        c += valid[q];
+    constexpr int HPT = HIST_MAX / FT;
+    __shared__ int win[HIST_MAX + 16];
+    __shared__ Small sm;
+    const int row = blockIdx.x, tid = threadIdx.x;
+    const int32_t *hist = nullptr, *drafts = nullptr;
+    int nd = 0;
+    if (a.direct) {
+        if (a.hist) hist = a.hist + (size_t)row * a.hist_len;
+    } else {
+        const int b = row < a.nrow_p ? row / (a.k + 1) : (row - a.nrow_p) / a.k;
+        nd = row < a.nrow_p ? row % (a.k + 1) : (row - a.nrow_p) % a.k;
+        if (a.hist) hist = a.hist + (size_t)b * a.hist_len;
+        drafts = a.draft + (size_t)b * a.k;
     }
+    if (tid < SWV) sm.scan[tid] = 0;           // (the block scan reads SWV wave sums)
+    if (tid == 0) sm.iv[0] = 0;
+    int tok[HPT], c = 0;
+#pragma unroll
+    for (int q = 0; q < HPT; q++) {
+        const int i = tid * HPT + q;
+        tok[q] = hist && i < a.hist_len ? hist[i] : -1;
+        c += tok[q] >= 0 ? 1 : 0;
+    }
+    __syncthreads();
     uint32_t L;
-    uint32_t p = block_excl_scan((uint32_t)c, sm, &L);
-    const int total = (int)L + nd, cap = P.penalty_last_n;
+    uint32_t p = block_excl_scan((uint32_t)c, &sm, &L);
+    const int total = (int)L + nd, cap = a.prm.penalty_last_n;
     const int start = total > cap ? total - cap : 0;
     const int wn = total - start;
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-        if (valid[q]) {
-            if ((int)p >= start) win[p - start] = hist[tid * 4 + q];
+    for (int q = 0; q < HPT; q++) {
+        if (tok[q] >= 0) {
+            if ((int)p >= start) win[p - start] = tok[q];
             p++;
         }
     }
-    for (int d = tid; d < nd; d += SB) {
+    for (int d = tid; d < nd; d += FT) {
         const int at = (int)L + d;
         if (at >= start) win[at - start] = drafts[d];
     }
-    strided(V, [&](int i) { return logits[i]; }, [&](int i, float l) { pen[i] = l; });
     __syncthreads();
-    for (int a = tid; a < wn; a += SB) {
-        const int tok = win[a];
-        if (tok < 0 || tok >= V) continue;
+    int2* out = (int2*)(a.e2 + (size_t)row * BAND);
+    static_assert(BAND / 2 >= HIST_MAX + 16, "the window's tokens fit");
+    for (int i = tid; i < wn; i += FT) {
+        const int t = win[i];
+        if (t < 0 || t >= a.V) continue;
         bool first = true;
         int count = 0;
+#pragma unroll 8
         for (int b = 0; b < wn; b++) {
-            if (win[b] == tok) {
-                if (b < a) first = false;
+            if (win[b] == t) {
+                if (b < i) first = false;
                 count++;
             }
         }
-        if (!first) continue;
-        float l = logits[tok];
-        if (l <= 0.0f) l *= P.penalty_repeat;
-        else l /= P.penalty_repeat;
-        const float sub = (float)count * P.penalty_freq;
-        l -= sub + P.penalty_present;
-        pen[tok] = l;
+        if (first) out[atomicAdd(&sm.iv[0], 1)] = int2{t, count};   // (applied in any order)
     }
     __syncthreads();
-    return pen;
+    if (tid == 0) a.st[row].wn = sm.iv[0];
 }
 
-// the logits row `row` of the build (penalties off)
-__device__ __forceinline__ const float* row_logits(const DistArgs& a, int row)
+// row `row` of the logits as given, and (the penalised copy when penalties
+// are on) as the build takes them
+__device__ __forceinline__ const float* row_given(const DistArgs& a, int row)
 {
     if (a.direct || row < a.nrow_p) return a.p_logits + (size_t)row * a.V;
     return a.q_logits + (size_t)(row - a.nrow_p) * a.V;
+}
+__device__ __forceinline__ const float* row_logits(const DistArgs& a, int row)
+{
+    return a.pen_on ? a.pen + (size_t)row * a.V : row_given(a, row);
 }
 
 // The split top-p build's first two launches, EXP_SPLIT workgroups per row:
@@ -1082,8 +1106,278 @@ __global__ __launch_bounds__(256) void fmap_kernel(DistArgs a)
     }
 }
 
+// What a build needs of the whole row before its candidates, EXP_SPLIT
+// workgroups per row (one workgroup streams a row at 60-100 GB/s, 6-10 us a
+// pass over 151,936 logits, and took five passes): the penalised copy and the
+// part's maximum, and for a top-k build (sel > 0) the part's keys down to its
+// sel-th largest.  Those are whole bins of a histogram over the keys' top 12
+// bits: the row's sel largest keys lie in the bins up to the smallest such
+// bin of any part (the part that has it holds sel keys there), and every part
+// has given all its keys in those.
+constexpr int PART_MAX = (VMAX / EXP_SPLIT + 3) & ~3, PIPT = (PART_MAX + FT - 1) / FT;
+// the part's elements of this thread, i0 + tid + q SB (loads issued together, at clamped indices)
+__device__ __forceinline__ void part_load(const float* lg, int i0, int i1, float (&v)[PIPT])
+{
+#pragma unroll
+    for (int q = 0; q < PIPT; q++) {
+        const int i = i0 + (int)threadIdx.x + q * FT;
+        v[q] = lg[i < i1 ? i : i0];
+    }
+}
+__global__ __launch_bounds__(FT) void front_kernel(DistArgs a)
+{
+    extern __shared__ __align__(16) unsigned char sdyn[];
+    float* x = (float*)sdyn;                   // (with penalties) the part's logits
+    __shared__ uint32_t hist[4096];
+    __shared__ Small sm;
+    const int part = blockIdx.y, row = blockIdx.x, V = a.V, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    DistState& st = a.st[row];
+    int i0, i1;
+    exp_part(V, part, &i0, &i1);
+    const int n = i1 - i0;
+    if (n <= 0) {                              // (the whole workgroup)
+        if (tid == 0) {
+            st.pmax[part] = -INFINITY;
+            st.fcnt[part] = 0;
+            st.fval[part] = 4095;
+        }
+        return;
+    }
+    float v[PIPT];
+    part_load(row_given(a, row), i0, i1, v);
+    if (tid == 0) {
+        sm.iv[0] = 4095;
+        sm.iv[1] = 0;
+    }
+    if (tid < SWV) sm.scan[tid] = 0;           // (the block scan reads SWV wave sums)
+#pragma unroll
+    for (int q = 0; q < 4096 / FT; q++) hist[tid + q * FT] = 0;
+    if (a.pen_on) {
+        const int wn = st.wn;
+        const int2* w = (const int2*)(a.e2 + (size_t)row * BAND);
+#pragma unroll
+        for (int q = 0; q < PIPT; q++)
+            if (tid + q * FT < n) x[tid + q * FT] = v[q];
+        __syncthreads();
+        for (int i = tid; i < wn; i += FT) {
+            const int2 t = w[i];
+            if (t.x < i0 || t.x >= i1) continue;
+            float l = x[t.x - i0];
+            if (l <= 0.0f) l *= a.prm.penalty_repeat;
+            else l /= a.prm.penalty_repeat;
+            const float sub = (float)t.y * a.prm.penalty_freq;
+            l -= sub + a.prm.penalty_present;
+            x[t.x - i0] = l;
+        }
+        __syncthreads();
+        float* pen = a.pen + (size_t)row * V + i0;
+#pragma unroll
+        for (int q = 0; q < PIPT; q++)
+            if (tid + q * FT < n) pen[tid + q * FT] = v[q] = x[tid + q * FT];
+    }
+    __syncthreads();
+    float mx = -INFINITY;
+#pragma unroll
+    for (int q = 0; q < PIPT; q++)
+        if (tid + q * FT < n) {
+            mx = fmaxf(mx, v[q]);
+            if (a.sel > 0) atomicAdd(&hist[desc_key(v[q]) >> 20], 1u);
+        }
+    mx = cpv_wave_reduce(mx, cpv_op_max());
+    if (lane == 0) sm.wf[wave] = mx;
+    __syncthreads();
+    if (tid == 0) {
+        for (int w = 1; w < FT / 64; w++) mx = fmaxf(mx, sm.wf[w]);
+        st.pmax[part] = mx;
+    }
+    if (a.sel <= 0) return;
+    constexpr int BPT = 4096 / FT;
+    uint32_t c[BPT], sum = 0, tot;
+#pragma unroll
+    for (int q = 0; q < BPT; q++) sum += c[q] = hist[tid * BPT + q];
+    uint32_t run = block_excl_scan(sum, &sm, &tot);
+#pragma unroll
+    for (int q = 0; q < BPT; q++) {
+        const uint32_t before = run;
+        run += c[q];
+        if (before < (uint32_t)a.sel && run >= (uint32_t)a.sel) sm.iv[0] = tid * BPT + q;   // (one bin)
+    }
+    __syncthreads();
+    const uint32_t bin = (uint32_t)sm.iv[0];
+    unsigned long long* out = a.bkeys + (size_t)row * BAND + part * FCAP;
+#pragma unroll
+    for (int q = 0; q < PIPT; q++)
+        if (tid + q * FT < n && desc_key(v[q]) >> 20 <= bin) {
+            const int at = atomicAdd(&sm.iv[1], 1);
+            if (at < FCAP) out[at] = cand_key(v[q], i0 + tid + q * FT);
+        }
+    __syncthreads();
+    if (tid == 0) {
+        st.fcnt[part] = sm.iv[1];
+        st.fval[part] = (int)bin;
+    }
+}
+
+// the row's maximum from its parts' (wave-uniform)
+__device__ __forceinline__ float parts_max(const DistState& st)
+{
+    const int lane = threadIdx.x & 63;
+    return cpv_wave_reduce(lane < EXP_SPLIT ? st.pmax[lane] : -INFINITY, cpv_op_max());
+}
+
+// A min-p build's candidates, after the parts' maxima: the keys not behind
+// the floor's (a NaN ranks before every number, so the set stays a prefix of
+// the candidate order), and the count of logits at or above it
+__global__ __launch_bounds__(FT) void floor_kernel(DistArgs a)
+{
+    __shared__ int s_n[2];
+    const int part = blockIdx.y, row = blockIdx.x, V = a.V, tid = threadIdx.x;
+    DistState& st = a.st[row];
+    int i0, i1;
+    exp_part(V, part, &i0, &i1);
+    if (i0 >= i1) {                            // (the whole workgroup)
+        if (tid == 0) st.fcnt[part] = st.fval[part] = 0;
+        return;
+    }
+    float v[PIPT];
+    part_load(row_logits(a, row), i0, i1, v);
+    const float floor_l = parts_max(st) + a.ln_min_p;
+    const uint32_t fk = desc_key(floor_l);
+    if (tid < 2) s_n[tid] = 0;
+    __syncthreads();
+    unsigned long long* out = a.bkeys + (size_t)row * BAND + part * FCAP;
+    int cnt = 0;
+#pragma unroll
+    for (int q = 0; q < PIPT; q++) {
+        const int i = i0 + tid + q * FT;
+        if (i >= i1) continue;
+        cnt += v[q] >= floor_l ? 1 : 0;
+        if (desc_key(v[q]) <= fk) {
+            const int at = atomicAdd(&s_n[0], 1);
+            if (at < FCAP) out[at] = cand_key(v[q], i);
+        }
+    }
+    cnt = cpv_wave_reduce(cnt, cpv_op_add());
+    if ((tid & 63) == 0 && cnt) atomicAdd(&s_n[1], cnt);
+    __syncthreads();
+    if (tid == 0) {
+        st.fcnt[part] = s_n[0];
+        st.fval[part] = s_n[1];
+    }
+}
+
+// The parts' selected keys narrowed to about M, sorted and written out as the
+// first candidates (emit_band's results): their number, at least M of them;
+// or 0 when a part selected more than it may keep or the M largest cannot be
+// told from more than a key per thread (the caller then emits bands).  The
+// keys with the M largest logits lie in the first bins of a histogram over
+// the selected keys' own range of desc_key (4096 bins).
+__device__ __noinline__ int emit_selected(const float* lg, const DistState* stp, const unsigned long long* src,
+                                          bool bins, int M, int32_t* sid, float* sl, unsigned long long* keys,
+                                          Small* sm)
+{
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const DistState& st = *stp;
+    const int fc = lane < EXP_SPLIT ? st.fcnt[lane] : 0, fv = lane < EXP_SPLIT ? st.fval[lane] : 4095;
+    if (M < 1 || __builtin_amdgcn_ballot_w64(fc > FCAP)) return 0;   // (the same in every wave)
+    // a wave takes part wave, then part wave + SWV
+    constexpr int KPL = FCAP / 64, PPW = EXP_SPLIT / SWV;
+    static_assert(PPW * SWV == EXP_SPLIT && KPL * 64 == FCAP, "whole parts per wave");
+    // (top-k: every part's keys are complete down to the smallest bin only)
+    const int bin = bins ? (int)-cpv_wave_reduce(-(float)fv, cpv_op_max()) : 4095;
+    unsigned long long k[PPW][KPL];
+    uint32_t lo = ~0u, hi = 0u;
+#pragma unroll
+    for (int p = 0; p < PPW; p++) {
+        const int part = wave + p * SWV;
+        const int n = __builtin_amdgcn_readlane(fc, __builtin_amdgcn_readfirstlane(part));
+#pragma unroll
+        for (int q = 0; q < KPL; q++) {
+            const int i = lane + 64 * q;
+            k[p][q] = src[part * FCAP + (i < n ? i : 0)];
+            if (i >= n || (int)(k[p][q] >> 52) > bin) k[p][q] = ~0ull;
+            if (k[p][q] != ~0ull) {
+                const uint32_t d = (uint32_t)(k[p][q] >> 32);
+                lo = d < lo ? d : lo;
+                hi = d > hi ? d : hi;
+            }
+        }
+    }
+    uint32_t* hist = (uint32_t*)(keys + SB);   // after the kept keys
+    int* place = (int*)hist;                   // (over the bins, once they are read)
+    __syncthreads();
+    for (int q = tid; q < 4096; q += SB) hist[q] = 0;
+    if (tid == 0) {
+        sm->iv[0] = 4095;
+        sm->iv[3] = 0;
+        sm->scan[0] = ~0u;
+        sm->scan[1] = 0;
+    }
+    __syncthreads();
+    atomicMin(&sm->scan[0], lo);
+    atomicMax(&sm->scan[1], hi);
+    __syncthreads();
+    lo = sm->scan[0];
+    hi = sm->scan[1];
+    if (lo > hi) return 0;                     // (no key)
+    const int sh = hi - lo < 4096u ? 0 : 20 - __builtin_clz(hi - lo);
+#pragma unroll
+    for (int p = 0; p < PPW; p++)
+#pragma unroll
+        for (int q = 0; q < KPL; q++)
+            if (k[p][q] != ~0ull) atomicAdd(&hist[((uint32_t)(k[p][q] >> 32) - lo) >> sh], 1u);
+    __syncthreads();
+    uint32_t c[4], sum = 0, tot;
+#pragma unroll
+    for (int q = 0; q < 4; q++) sum += c[q] = hist[tid * 4 + q];
+    uint32_t run = block_excl_scan(sum, sm, &tot);
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const uint32_t before = run;
+        run += c[q];
+        if (before < (uint32_t)M && run >= (uint32_t)M) sm->iv[0] = tid * 4 + q;   // (one bin)
+    }
+    __syncthreads();
+    const uint32_t last = (uint32_t)sm->iv[0];
+    place[tid] = 0;
+#pragma unroll
+    for (int p = 0; p < PPW; p++)
+#pragma unroll
+        for (int q = 0; q < KPL; q++)
+            if (k[p][q] != ~0ull && ((uint32_t)(k[p][q] >> 32) - lo) >> sh <= last) {
+                const int at = atomicAdd(&sm->iv[3], 1);
+                if (at < SB) keys[at] = k[p][q];
+            }
+    __syncthreads();
+    // a key's place is the number of keys before it (they are distinct),
+    // counted by as many threads per key as there are
+    const int cnt = sm->iv[3];
+    if (cnt > SB || cnt < M) return 0;
+    const int gs = (cnt + 63) & ~63, ng = SB / gs, grp = tid / gs, kk = tid - grp * gs;
+    const unsigned long long key = keys[kk < cnt ? kk : 0];
+    if (grp < ng) {                            // (wave-uniform)
+        const int per = (cnt + ng - 1) / ng, q1 = min(cnt, (grp + 1) * per);
+        int at = 0;
+#pragma unroll 4
+        for (int q = grp * per; q < q1; q++) at += keys[q] < key ? 1 : 0;
+        if (kk < cnt && at) atomicAdd(&place[kk], at);
+    }
+    __syncthreads();
+    if (tid < cnt) {
+        const int id = (int)(key & 0x3ffffull), at = place[tid];
+        sid[at] = id;
+        sl[at] = lg[id];
+    }
+    __syncthreads();
+    return cnt;
+}
+
 // Sampler::build for one row (lib.rs:229-376), leaving the distribution as
 // n candidates (sid, sl, pr) in candidate order.
+// PH: 0 the whole build; 1 (two workgroups per row) and 2 the split top-p
+// build; 3 a top-k or min-p build whose candidates were selected by parts.
+// (A kernel each: one for all phases held 86 spilled registers.)
+template <int PH>
 __global__ __launch_bounds__(SB) void dist_kernel(DistArgs a)
 {
     extern __shared__ __align__(16) unsigned char sdyn[];
@@ -1094,40 +1388,16 @@ __global__ __launch_bounds__(SB) void dist_kernel(DistArgs a)
     // phase 1 workgroup 2 r sums row r's exponentials in index order while
     // workgroup 2 r + 1 emits its first band (the two need nothing from each
     // other); phase 2 goes on from both
-    const int tid = threadIdx.x, row = a.phase == 1 ? (int)(blockIdx.x >> 1) : (int)blockIdx.x, V = a.V;
-    const int role = a.phase == 1 ? (int)(blockIdx.x & 1) : 0;
+    const int tid = threadIdx.x, row = PH == 1 ? (int)(blockIdx.x >> 1) : (int)blockIdx.x, V = a.V;
+    const int role = PH == 1 ? (int)(blockIdx.x & 1) : 0;
     const cpv_sampler_params& P = a.prm;
-    const float* logits;
-    const int32_t* hist = nullptr;
-    const int32_t* drafts = nullptr;
-    int nd = 0;
-    if (a.direct) {
-        logits = a.p_logits + (size_t)row * V;
-        if (a.hist) hist = a.hist + (size_t)row * a.hist_len;
-    } else {
-        int b, j;
-        if (row < a.nrow_p) {
-            b = row / (a.k + 1);
-            j = row % (a.k + 1);
-            logits = a.p_logits + (size_t)row * V;
-        } else {
-            const int r = row - a.nrow_p;
-            b = r / a.k;
-            j = r % a.k;
-            logits = a.q_logits + (size_t)r * V;
-        }
-        if (a.hist) hist = a.hist + (size_t)b * a.hist_len;
-        drafts = a.draft + (size_t)b * a.k;
-        nd = j;
-    }
     const size_t off = (size_t)row * V;
     int32_t* sid = a.sid + off;
     float* sl = a.sl + off;
     float* pr = a.pr + off;
-    const float* lg = logits;
-    if (a.pen_on) lg = apply_penalties(logits, a.pen + off, V, hist, a.hist_len, drafts, nd, P, (int*)keys, sm);
+    const float* lg = row_logits(a, row);
 
-    if (P.temp <= 0.0f) {                                  // :324-337 point mass at the first maximum
+    if (PH == 0 && P.temp <= 0.0f) {                                  // :324-337 point mass at the first maximum
         const int best = block_argmax([&](int i) { return lg[i]; }, V, 0, sm);
         if (tid == 0) {
             sid[0] = best;
@@ -1138,14 +1408,20 @@ __global__ __launch_bounds__(SB) void dist_kernel(DistArgs a)
         return;
     }
 
-    const bool top_k = P.top_k > 0 && P.top_k < V;         // :272-280
-    const bool min_p = !top_k && P.min_p > 0.0f;           // :281-295
-    const bool top_p = !top_k && !min_p && P.top_p < 1.0f; // :296-316
+    constexpr bool split = PH == 1 || PH == 2;
+    const bool top_k = !split && P.top_k > 0 && P.top_k < V;         // :272-280
+    const bool min_p = !split && !top_k && P.min_p > 0.0f;           // :281-295
+    const bool top_p = PH == 3 ? false : split || (!top_k && !min_p && P.top_p < 1.0f); // :296-316
     // (the split build needs no maximum here: exp_kernel has used it, and
     // top-p's final softmax is relative to the first candidate)
-    const float mx = a.phase != 0 || a.pre_exp ? 0.0f : block_max([&](int i) { return lg[i]; }, V, sm);
+    float mx = 0.0f;
+    if (PH == 3 && a.sel < 0) {
+        mx = parts_max(a.st[row]);
+    } else if (PH == 0 && !a.pre_exp && !top_k) {
+        mx = block_max([&](int i) { return lg[i]; }, V, sm);
+    }
     int n;
-    if (top_k || min_p || top_p) {
+    if (PH != 0 || top_k || min_p || top_p) {
         int M = 0, emitted = 0;
         unsigned long long last = 0;
         if (top_k) {
@@ -1153,7 +1429,8 @@ __global__ __launch_bounds__(SB) void dist_kernel(DistArgs a)
             if (M > V) M = V;
         } else if (min_p) {
             const float floor_l = mx + a.ln_min_p;
-            M = block_count([&](int i) { return lg[i] >= floor_l; }, V, sm);
+            if (PH == 3 && a.sel < 0) M = cpv_wave_reduce((tid & 63) < EXP_SPLIT ? a.st[row].fval[tid & 63] : 0, cpv_op_add());
+            else M = block_count([&](int i) { return lg[i] >= floor_l; }, V, sm);
         } else {
             // softmax over the vocabulary in index order, then the probe:
             // the smallest of 1024, 8192, ... (capped at V) whose sorted
@@ -1163,7 +1440,7 @@ __global__ __launch_bounds__(SB) void dist_kernel(DistArgs a)
             // final probabilities overwrite it at the end)
             float sum1 = 0.0f;
             int cnt;
-            if (a.phase == 2) {
+            if (PH == 2) {
                 sum1 = a.st[row].sum1;
                 cnt = a.st[row].cnt;
                 last = a.st[row].last;
@@ -1198,12 +1475,12 @@ __global__ __launch_bounds__(SB) void dist_kernel(DistArgs a)
                         stage_head(pv, V, fl);
                         sum1 = block_fold(pv, V, 0.0f, 0.0f, F_NONE, sm, FOLD_SEQ, fl->head).sum;
                     }
-                    if (a.phase == 1) {
+                    if (PH == 1) {
                         if (tid == 0) a.st[row].sum1 = sum1;
                         return;
                     }
                 }
-                if (a.phase == 1) {
+                if (PH == 1) {
                     // the band's keys in parts for band_part_kernel to sort,
                     // or the band sorted here
                     DistState& st = a.st[row];
@@ -1227,7 +1504,7 @@ __global__ __launch_bounds__(SB) void dist_kernel(DistArgs a)
             }
             float s = 0.0f;
             int ifirst = -1;
-            if (a.phase == 2 && a.st[row].np > 0 && cnt > 0) {
+            if (PH == 2 && a.st[row].np > 0 && cnt > 0) {
                 // the first band in parts: each part's composed step where it
                 // applies and leaves the sum below top_p (the fold's values
                 // only grow, so no element of the part meets the predicate),
@@ -1282,6 +1559,7 @@ __global__ __launch_bounds__(SB) void dist_kernel(DistArgs a)
                 if (keep <= probe) M = keep;
             }
         }
+        if (PH == 3) emitted = emit_selected(lg, a.st + row, a.bkeys + (size_t)row * BAND, a.sel > 0, M, sid, sl, keys, sm);
         while (emitted < M) {
             const int cnt = emit_band(lg, V, emitted > 0, &last, M - emitted, emitted, sid, sl, keys, sm);
             if (cnt <= 0) break;
@@ -1321,9 +1599,9 @@ __global__ __launch_bounds__(SB) void dist_kernel(DistArgs a)
     }
     // :371-374 temperature, then softmax over the survivors (:461-471)
     const float T = P.temp;
-    const float mx2 = (top_k || min_p || top_p ? sl[0] : mx) / T;
+    const float mx2 = (PH != 0 || top_k || min_p || top_p ? sl[0] : mx) / T;
     __syncthreads();
-    if (top_p && a.phase == 2 && a.st[row].np > 0 && n <= a.st[row].cnt) {
+    if (top_p && PH == 2 && a.st[row].np > 0 && n <= a.st[row].cnt) {
         // the survivors lie in the first band: its parts' e2 and composed
         // steps (band_part_kernel), the steps where they apply, whole parts
         // below n; the rest element by element
@@ -1701,30 +1979,39 @@ cpv_status dist_launch(cpv_ctx* ctx, DistArgs& a, int rows)
     const size_t lds = SAMPLE_LDS_KEYS + sizeof(Small) + sizeof(FoldLds);
     if (lds > ctx->lds_max) return cpv_fail(ctx, CPV_EUNSUPPORTED, "sampler: needs %zu bytes of LDS", lds);
     const int e0 = cpv_prof_mark(ctx);
-    // top-p without penalties: the maximum and the exponentials over
+    // penalties: the penalised rows first (front_kernel).  Top-p: the maximum and the exponentials over
     // EXP_SPLIT workgroups per row; then, when two workgroups per row fit the
     // CUs, the index-order sum and the first band side by side (two
     // workgroups per row), then the rest
     const cpv_sampler_params& P = a.prm;
     const bool top_k = P.top_k > 0 && P.top_k < a.V;
-    a.pre_exp = P.temp > 0.0f && !top_k && !(P.min_p > 0.0f) && P.top_p < 1.0f && !a.pen_on;
+    a.pre_exp = P.temp > 0.0f && !top_k && !(P.min_p > 0.0f) && P.top_p < 1.0f && rows <= 65535 &&
+                (!a.pen_on || 2 * rows <= ctx->cu_count);
+    // top-k and min-p: the candidates selected by parts of the row first
+    // (top-k up to FRONT_K of them: a part may keep FCAP keys)
+    const int kk = P.top_k > P.min_keep ? P.top_k : P.min_keep;
+    a.sel = P.temp > 0.0f ? top_k ? (kk <= FRONT_K ? kk : 0) : P.min_p > 0.0f ? -1 : 0 : 0;
+    if (a.pen_on || a.sel) {
+        if (a.pen_on) window_kernel<<<(unsigned)rows, FT, 0, ctx->stream>>>(a);
+        const size_t part_b = a.pen_on ? (size_t)(((a.V + EXP_SPLIT - 1) / EXP_SPLIT + 3) & ~3) * 4 : 0;
+        front_kernel<<<dim3((unsigned)rows, EXP_SPLIT), FT, part_b, ctx->stream>>>(a);
+    }
+    if (!a.pen_on && !a.sel && a.pre_exp) rowmax_part_kernel<<<dim3(EXP_SPLIT, (unsigned)rows), 256, 0, ctx->stream>>>(a);
+    if (a.sel < 0) floor_kernel<<<dim3((unsigned)rows, EXP_SPLIT), FT, 0, ctx->stream>>>(a);
     if (a.pre_exp) {
-        rowmax_part_kernel<<<dim3(EXP_SPLIT, (unsigned)rows), 256, 0, ctx->stream>>>(a);
         exp_kernel<<<dim3(EXP_SPLIT, (unsigned)rows), 256, 0, ctx->stream>>>(a);
         fmap_kernel<<<dim3(EXP_SPLIT, (unsigned)rows), 256, 0, ctx->stream>>>(a);
     }
     if (a.pre_exp && 2 * rows <= ctx->cu_count) {
         // the first band in parts while the part workgroups fit the CUs two to a CU
         a.parts = rows * MAXP <= 2 * ctx->cu_count;
-        a.phase = 1;
-        dist_kernel<<<(unsigned)(2 * rows), SB, lds, ctx->stream>>>(a);
+        dist_kernel<1><<<(unsigned)(2 * rows), SB, lds, ctx->stream>>>(a);
         if (a.parts)
             band_part_kernel<<<dim3(MAXP, (unsigned)rows), SB, PART_LDS_KEYS + sizeof(Small), ctx->stream>>>(a);
-        a.phase = 2;
-        dist_kernel<<<(unsigned)rows, SB, lds, ctx->stream>>>(a);
+        dist_kernel<2><<<(unsigned)rows, SB, lds, ctx->stream>>>(a);
     } else {
-        a.phase = 0;
-        dist_kernel<<<(unsigned)rows, SB, lds, ctx->stream>>>(a);
+        if (a.sel) dist_kernel<3><<<(unsigned)rows, SB, lds, ctx->stream>>>(a);
+        else dist_kernel<0><<<(unsigned)rows, SB, lds, ctx->stream>>>(a);
     }
     CPV_HIP(ctx, hipGetLastError());
     cpv_prof_add(ctx, e0, CPV_PROF_SAMPLE, (double)rows * a.V * 4.0);

@@ -80,6 +80,34 @@ def test_distribution_headline_rows(ctx, name):
     check_dist(ctx, logits, cpvo.SamplerParams(**DIST_CASES[name]))
 
 
+# top-k and min-p candidates are selected by 32 parts of a row: vocabularies
+# below the parts' count and at their edges, counts up to and past what a part
+# selects, ties across parts, and rows whose parts select too many (equal
+# logits), which take the bands instead
+SELECT_CASES = [dict(temp=0.7, top_k=1), dict(temp=0.8, top_k=40), dict(temp=0.8, top_k=256, top_p=0.9),
+                dict(temp=0.8, top_k=257), dict(temp=0.9, top_k=3, min_keep=70), dict(temp=0.9, min_p=0.05),
+                dict(temp=0.9, min_p=1.0), dict(temp=1.1, min_p=1e-4, top_p=0.8),
+                dict(temp=0.8, top_k=40, min_p=0.05, penalty_repeat=1.3, penalty_freq=0.1),
+                dict(temp=0.8, min_p=0.02, penalty_repeat=1.2), dict(temp=0.8, top_p=0.9, penalty_repeat=1.2),
+                dict(temp=0.0, penalty_repeat=1.5)]
+
+
+@pytest.mark.parametrize("v", [2, 31, 33, 129, 4097, 20000, 262144])
+def test_distribution_selected_by_parts(ctx, v):
+    rng = np.random.default_rng(v)
+    x = spiked(rng, (6, v))
+    x[1] = np.round(x[1])                            # ties
+    x[2] = 0.25                                      # all equal
+    x[3] = np.where(rng.random(v) < 0.5, -0.0, 0.0)  # equal but for the sign of zero
+    x[4, rng.random(v) < 0.3] = -np.inf              # banned tokens
+    x[4, 0] = 1.0
+    x[5, :v // 2] -= 40.0                            # every candidate in some of the parts
+    hist = rng.integers(-1, v, size=(6, 40)).astype(np.int32)
+    for c in SELECT_CASES:
+        print(f"case v={v} {c}", flush=True)
+        check_dist(ctx, x, cpvo.SamplerParams(**c), hist if "penalty_repeat" in c else None)
+
+
 @pytest.mark.parametrize("rows", [60, 140])
 def test_distribution_top_p_row_counts(ctx, rows):
     # top-p builds: the maximum and exponentials over many workgroups per
