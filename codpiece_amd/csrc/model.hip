@@ -290,7 +290,8 @@ constexpr int RW = RB / 64;  // most waves
 constexpr int RUU = 3;       // most units per wave: rows up to 3 * 16 * 256 = 12288 elements
 constexpr int RQ = RUU * 4;  // most register slots per thread
 
-enum { SRC_X = 0, SRC_ADD = 1, SRC_SET = 2, SRC_GATE = 3, SRC_SWIGLU = 4, SRC_GATE_FOLD = 5, SRC_CAT = 6 };
+enum { SRC_X = 0, SRC_ADD = 1, SRC_SET = 2, SRC_GATE = 3, SRC_SWIGLU = 4, SRC_GATE_FOLD = 5, SRC_CAT = 6,
+       SRC_SWIGLU_Y = 7 };
 constexpr int FOLD_MAX = 512;   // attention chunks a SRC_GATE_FOLD row kernel folds (contexts to 64k)
 
 struct RowArgs {
@@ -298,6 +299,7 @@ struct RowArgs {
     float* x;              // residual rows [T][xs] (SRC_X / _ADD / _SET read and write it)
     int64_t xs;
     cpv_gout g;            // kept GEMM result (SRC_ADD / _SET / _SWIGLU)
+    const float* gu;       // SRC_SWIGLU_Y: the gate|up outputs [T][2 n]
     const float* att;      // SRC_GATE: attention output [T][n] and gate [T][n]
     const float* gate;
     cpv_attn_part part;    // SRC_GATE_FOLD: the attention's chunk partials (rows = T * n / hd)
@@ -539,7 +541,7 @@ __global__ __launch_bounds__(RB) void row_kernel(RowArgs a)
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
                     const int vq = (int)rintf(iscale * x[k]);
-                    q[k] = (int8_t)(vq < 127 ? vq : 127);   // (the code as stored: what the sums add)
+                    q[k] = vq < 127 ? vq : 127;
                 }
                 d = 1.0f / iscale;
             } else {
@@ -570,7 +572,8 @@ __global__ __launch_bounds__(RB) void row_kernel(RowArgs a)
 }
 
 // The same for rows that need no row-wide reduction: the gated attention
-// output (SRC_GATE) and SwiGLU of a kept gate|up result (SRC_SWIGLU), each
+// output (SRC_GATE) and SwiGLU of a kept gate|up result (SRC_SWIGLU; of its
+// stored outputs: SRC_SWIGLU_Y), each
 // quantized for the next GEMM.  One 256-thread block per (unit, row).
 template <int SRC>
 __global__ __launch_bounds__(256) void unit_kernel(RowArgs a)
@@ -653,6 +656,13 @@ __global__ __launch_bounds__(256) void unit_kernel(RowArgs a)
         const float gv = a.gate[(int64_t)m * n + ec], at = a.att[(int64_t)m * n + ec];
         const float sig = 1.0f / (1.0f + cpv_expf(-gv));
         val = e < n ? at * sig : 0.0f;
+    } else if (SRC == SRC_SWIGLU_Y) {
+        const float* gu = a.gu + (int64_t)m * 2 * n;
+        const float gv = gu[ec], uv = gu[n + ec];
+        if (e < n) {
+            const float sl = gv / (1.0f + cpv_expf(-gv));
+            val = sl * uv;
+        }
     } else {
         double* acc = a.g.acc + (int64_t)m * a.g.n_pad;
         const double S0 = acc[ec], S1 = acc[n + ec];
@@ -691,7 +701,7 @@ __global__ __launch_bounds__(256) void unit_kernel(RowArgs a)
         if (ax > 0.0f) {
             const float iscale = -127.0f / sx;
             const int vq = (int)rintf(iscale * val);
-            q = (int8_t)(vq < 127 ? vq : 127);   // (the code as stored: what the sums add)
+            q = vq < 127 ? vq : 127;
             d = 1.0f / iscale;
         }
         qa[(int64_t)m * Kp + e] = (int8_t)q;
@@ -1275,6 +1285,7 @@ cpv_status row_launch(cpv_ctx* ctx, const RowArgs& a, int T)
             return cpv_fail(ctx, CPV_EUNSUPPORTED, "gate fold: head dim %d, %d chunks", a.hd, a.part.nchunk);
         unit_kernel<SRC_GATE_FOLD><<<ugrid, 256, 0, ctx->stream>>>(a);
         break;
+    case SRC_SWIGLU_Y: unit_kernel<SRC_SWIGLU_Y><<<ugrid, 256, 0, ctx->stream>>>(a); break;
     default: unit_kernel<SRC_SWIGLU><<<ugrid, 256, 0, ctx->stream>>>(a); break;
     }
     CPV_HIP(ctx, hipGetLastError());
@@ -1544,11 +1555,20 @@ cpv_status block(cpv_session* s, const LayerW& L, float* x, int T, int64_t rope_
     r3.quant = 1;
     cpv_act_layout(L.gate_up->type, T, E, next_act(s), &r3.act);
     if ((st = row_launch(ctx, r3, T))) return st;
-    if ((st = cpv_qgemm_keep(ctx, L.gate_up, &r3.act, &g))) return st;
-    // SwiGLU, the down input
+    // SwiGLU, the down input.  The wide kernels write their outputs, f32 once
+    // (a kept result is f64 out, in and back to zero: the SwiGLU over 512 rows
+    // of 2 x 17408 took about 57 us; 34 -> 23 averaged over a
+    // prompt's chunks of 512 and 64 rows)
     RowArgs r4{};
-    r4.src = SRC_SWIGLU;
-    r4.g = g;
+    if (cpv_qgemm_wide_ok(L.gate_up, T) && L.gate_up->n == 2 * F) {
+        if ((st = cpv_qgemm_act(ctx, L.gate_up, &r3.act, s->gu))) return st;
+        r4.src = SRC_SWIGLU_Y;
+        r4.gu = s->gu;
+    } else {
+        if ((st = cpv_qgemm_keep(ctx, L.gate_up, &r3.act, &g))) return st;
+        r4.src = SRC_SWIGLU;
+        r4.g = g;
+    }
     r4.n = (int)F;
     r4.quant = 1;
     cpv_act_layout(L.down->type, T, F, next_act(s), &r4.act);
@@ -1566,8 +1586,8 @@ cpv_status project(cpv_session* s, const cpv_weight* w, const float* x, int T, f
 
 // x (+ a kept result) -> RMS norm with w -> y (f32) and the input of head w_head,
 // whose logits go to logits
-// rms(x) with weight w into y, then the head's logits; with keep, the head's
-// result stays in the accumulator (*keep, for cpv_argmax_peak_rows to
+// rms(x) with weight w into y, then the head's logits; with keep, a skinny
+// head's result stays in the accumulator (*keep, for cpv_argmax_peak_rows to
 // finalize), else keep->acc is null and the logits are stored
 cpv_status norm_head(cpv_session* s, float* x, int T, const cpv_gout* pend, const float* w, float* y,
                      const cpv_weight* w_head, float* logits, cpv_gout* keep = nullptr)
@@ -1594,7 +1614,10 @@ cpv_status norm_head(cpv_session* s, float* x, int T, const cpv_gout* pend, cons
     cpv_act_layout(w_head->type, T, hp.n_embd, next_act(s), &r.act);
     cpv_status st = row_launch(m->ctx, r, T);
     if (st != CPV_OK) return st;
-    if (keep) return cpv_qgemm_keep(m->ctx, w_head, &r.act, keep);
+    // (the wide kernels write the logits themselves: f32 once, where a kept
+    // result is f64 out, in and back to zero: the argmax's first pass over 64
+    // rows of 151,936 took 39 us)
+    if (keep && !cpv_qgemm_wide_ok(w_head, T)) return cpv_qgemm_keep(m->ctx, w_head, &r.act, keep);
     return cpv_qgemm_act(m->ctx, w_head, &r.act, logits);
 }
 

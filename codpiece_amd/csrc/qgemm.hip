@@ -73,7 +73,7 @@ __global__ __launch_bounds__(256) void quant_q8k_kernel(const float* __restrict_
     if (amax > 0.0f) {
         const float iscale = -127.0f / sx[imax];
         const int vq = (int)rintf(iscale * v);
-        q = (int8_t)(vq < 127 ? vq : 127);   // (the code as stored: what the sums below add)
+        q = vq < 127 ? vq : 127;
         d = 1.0f / iscale;
     }
     const int64_t Kp = (int64_t)U * 256;

@@ -251,9 +251,12 @@ __global__ __launch_bounds__(WT) __attribute__((amdgpu_waves_per_eu(wide_per_cu(
     };
     auto stage_store = [&](int buf, const Stage& t) {
         if constexpr (Q4) {
+            // (a sum's low 16 bits: a unit whose largest value is below 127 /
+            // FLT_MAX has out-of-range codes, stored as 0 or 127 but summed as
+            // 32-bit integers, which agree in those bits)
             v8h h;
 #pragma unroll
-            for (int i = 0; i < 8; i++) h[i] = (_Float16)(float)t.b[i >> 2][i & 3];
+            for (int i = 0; i < 8; i++) h[i] = (_Float16)(float)(short)t.b[i >> 2][i & 3];
             *(v8h*)&s.bs[buf][brow][8 * (tid & 1)] = h;
         }
         s.dad[buf][drow] = (double)t.d * s.sm[drow];

@@ -120,6 +120,24 @@ def test_qgemm_wide_row_blocks(ctx, tname, m):
     assert np.array_equal(y.view(np.uint32), ref.view(np.uint32)), np.abs(y - ref).max()
 
 
+@pytest.mark.parametrize("m", [5, 40])
+def test_qgemm_units_below_the_scale_range(ctx, m):
+    # a unit whose largest value is below 127 / FLT_MAX has an infinite inverse
+    # scale: its term is zero, on the skinny path and on the wide one's f16 sums
+    t, n, k = cpvo.Q4_K, 70, 1024
+    wq = weights(t, n, k)
+    x = np.random.default_rng(9).normal(0, 1, size=(m, k)).astype(np.float32)
+    x[1, 256:512] *= np.float32(1e-38)
+    x[2, :256] = np.float32(-3e-39)
+    w = ctx.upload_weight(t, wq, n, k)
+    y = ctx.qgemm(w, torch.from_numpy(x).cuda()).cpu().numpy()
+    w.free()
+    z = x.copy()
+    z[1, 256:512] = 0
+    z[2, :256] = 0
+    assert np.array_equal(y, cpvo.qgemm(t, wq, z))
+
+
 @pytest.mark.parametrize("tname", ["q4_k", "q6_k", "q8_0"])
 def test_qgemm_wide_whole_and_sliced(ctx, tname):
     # more (tile, row block) pairs than workgroups in flight: whole rounds run
