@@ -301,10 +301,12 @@ void cpv_act_layout(int type, int64_t m, int64_t k, void* buf, cpv_act* out);
 cpv_status cpv_quant_act(cpv_ctx* ctx, int type, const float* x, int64_t m, int64_t k, void* buf, cpv_act* out);
 cpv_status cpv_qgemm_act(cpv_ctx* ctx, const cpv_weight* w, const cpv_act* act, float* y);
 
-// The GEMMs for many activation rows (qgemm_wide.hip): the same accumulator
-// sums as cpv_qgemm_act's skinny kernels, on the 16x16x32 int8 MFMA, for all
-// act->m rows in one launch; cpv_qgemm_act takes them above 16 rows for
-// Q4_K and above 8 for Q6_K and Q8_0 (cpv_qgemm_wide_ok).
+// The GEMMs for many activation rows (qgemm_wide.hip): the same sums as
+// cpv_qgemm_act's skinny kernels, on the 16-row int8 MFMAs, for all act->m
+// rows in one launch, as outputs y [act->m][w->n] or, with y null, in the
+// accumulator gsum (zero on entry; left zero when y is given);
+// cpv_qgemm_act takes them above 16 rows for Q4_K and above 8 for Q6_K and
+// Q8_0 (cpv_qgemm_wide_ok).
 bool cpv_qgemm_wide_ok(const cpv_weight* w, int64_t m);
 cpv_status cpv_qgemm_wide(cpv_ctx* ctx, const cpv_weight* w, const cpv_act* act, double* gsum, int win, float* y);
 

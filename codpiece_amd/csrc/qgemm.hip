@@ -625,7 +625,7 @@ __global__ __launch_bounds__((64 * gemm_waves<TYPE, MC>())) void qgemm_kernel(Ge
 // v_mfma_i32_16x16x32_i8: one MFMA per (16-row block rb of the tile,
 // 32-element sub-block s of the unit) takes all 16 activation rows at once,
 // 32 MFMAs per item where the 4x4x4 shape needs 256 (the same layout as
-// qgemm_wide_kernel: A row and B column = lane % 16, codes 8 (lane / 16) ..
+// the wide kernels: A row and B column = lane % 16, codes 8 (lane / 16) ..
 // + 7 of the sub-block per lane, D rows 4 (lane / 16) + i of column lane %
 // 16).  Lane (c, g) = (lane % 16, lane / 16) thus holds the dots of
 // activation rows 4g..4g+3 with weight rows 16 rb + c, rb = 0..3: it decodes

@@ -677,11 +677,10 @@ namespace {
 // pairs 55; 5120 x 17408 at 256 rows: 8 blocks in 160 pairs x 3 slices 112, 4
 // in 320 whole pairs 146; Q8_0 7168 x 5120 at 201 rows: 3 blocks in 560 pairs
 // 75, 2 in 784 pairs 63.
-void wide_split(WideArgs& a, bool q80, int cus, int* nmt_out)
+void wide_split(WideArgs& a, bool q80, int maxb, int cus, int* nmt_out)
 {
     const int nb16 = (a.M + 15) / 16;
     double best = 1e30;
-    const int maxb = q80 ? MAX_NMT_Q80 : MAX_NMT;
     for (int mb = (nb16 + maxb - 1) / maxb; mb <= nb16; mb++) {
         const int nmt = (nb16 + mb - 1) / mb;
         if ((nb16 + nmt - 1) / nmt != mb) continue;   // (the same blocks in fewer workgroups)
@@ -742,7 +741,10 @@ cpv_status cpv_qgemm_wide(cpv_ctx* ctx, const cpv_weight* w, const cpv_act* act,
     if ((w->type != CPV_Q4_K && !q80 && !q6k) || act->kq == q80 || act->U != (int)w->units || act->m < 1 ||
         act->m > INT32_MAX / 2)
         return cpv_fail(ctx, CPV_EINVAL, "qgemm_wide: weight or activation format not supported");
-    if (16LL * MAX_NMT * act->U * 256 > INT32_MAX)   // the staging offsets within a row block are 32-bit
+    // (the staging offsets within a row block are 32-bit: very long rows in smaller blocks)
+    int maxb = q80 ? MAX_NMT_Q80 : MAX_NMT;
+    while (maxb > 0 && 16LL * maxb * act->U * 256 > INT32_MAX) maxb--;
+    if (maxb == 0)
         return cpv_fail(ctx, CPV_EUNSUPPORTED, "qgemm_wide: k=%lld too long", (long long)w->k);
     WideArgs a;
     a.w = (const uint8_t*)w->data;
@@ -763,7 +765,7 @@ cpv_status cpv_qgemm_wide(cpv_ctx* ctx, const cpv_weight* w, const cpv_act* act,
     if ((int64_t)a.tiles * ((a.M + 15) / 16) > INT32_MAX / 1024)
         return cpv_fail(ctx, CPV_EUNSUPPORTED, "qgemm_wide: %d tiles by %d rows", a.tiles, a.M);
     int nmt = 4;
-    wide_split(a, q80, ctx->cu_count, &nmt);
+    wide_split(a, q80, maxb, ctx->cu_count, &nmt);
     const int64_t blocks = (int64_t)a.tiles * a.mblocks;
     const int64_t rest = blocks - a.nfull, grid = a.nfull + rest * a.ksplit;
     const int ev = cpv_prof_mark(ctx);

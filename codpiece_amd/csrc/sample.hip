@@ -1979,16 +1979,20 @@ cpv_status dist_launch(cpv_ctx* ctx, DistArgs& a, int rows)
     const size_t lds = SAMPLE_LDS_KEYS + sizeof(Small) + sizeof(FoldLds);
     if (lds > ctx->lds_max) return cpv_fail(ctx, CPV_EUNSUPPORTED, "sampler: needs %zu bytes of LDS", lds);
     const int e0 = cpv_prof_mark(ctx);
-    // penalties: the penalised rows first (front_kernel).  Top-p: the maximum and the exponentials over
-    // EXP_SPLIT workgroups per row; then, when two workgroups per row fit the
-    // CUs, the index-order sum and the first band side by side (two
-    // workgroups per row), then the rest
+    // Penalties: the penalised rows first (front_kernel).  Top-p: the maximum
+    // and the exponentials over EXP_SPLIT workgroups per row; then, when two
+    // workgroups per row fit the CUs, the index-order sum and the first band
+    // side by side (two workgroups per row), then the rest.  (Penalised rows
+    // past that: 240 rows 720 us with the exponentials ahead, 617 without.)
     const cpv_sampler_params& P = a.prm;
     const bool top_k = P.top_k > 0 && P.top_k < a.V;
     a.pre_exp = P.temp > 0.0f && !top_k && !(P.min_p > 0.0f) && P.top_p < 1.0f && rows <= 65535 &&
                 (!a.pen_on || 2 * rows <= ctx->cu_count);
-    // top-k and min-p: the candidates selected by parts of the row first
-    // (top-k up to FRONT_K of them: a part may keep FCAP keys)
+    // Top-k and min-p: the candidates selected by parts of the row first, at
+    // every row count (V 151936, k = 4, us a call against one workgroup a
+    // row: top-k 40 at 9 rows 112 -> 52, at 240 rows 182 -> 156; min-p 129 ->
+    // 54 and 215 -> 138); top-k up to FRONT_K, as a part may keep FCAP keys
+    // and whole bins come with them (300: the bands, 107 us at 9 rows)
     const int kk = P.top_k > P.min_keep ? P.top_k : P.min_keep;
     a.sel = P.temp > 0.0f ? top_k ? (kk <= FRONT_K ? kk : 0) : P.min_p > 0.0f ? -1 : 0 : 0;
     if (a.pen_on || a.sel) {
