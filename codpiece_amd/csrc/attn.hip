@@ -788,7 +788,12 @@ cpv_status attn_block(cpv_ctx* ctx, const float* q, const uint16_t* kc, const ui
     // Over the API's f16 caches, 49 to 80 rows (a 16-node tree's) go in one
     // 80-row block: the chunk's K and V are loaded and converted to limbs
     // once for all of them, not once per 48-row block.
-    const bool wide = LR > QB_CHAIN && (int64_t)nchunk * Hkv >= 512;
+    // A prompt chunk's many rows over limb caches take 48-row blocks from 16
+    // chunks on too, at d = 128 (40/8 heads, 512 tokens after 3584: 429 -> 411
+    // us, 24/4: 268 -> 258; after 1000, 9 to 12 chunks, no gain; at d = 64
+    // 32/4: 222 -> 233).
+    const bool many = D == 128 && vl && LR >= 1024 && nchunk >= 16;
+    const bool wide = many || (LR > QB_CHAIN && (int64_t)nchunk * Hkv >= 512);
     const bool tree_blk = wide && !vl && LR > QB_WIDE && LR <= QB_TREE;
     const int QB = tree_blk ? QB_TREE : wide ? QB_WIDE : QB_CHAIN;
     const dim3 cgrid((unsigned)(nchunk * Hkv), 1u, (unsigned)((LR + QB - 1) / QB));

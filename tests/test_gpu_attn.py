@@ -67,11 +67,12 @@ def test_27b_class_chain(ctx, n_past):
 
 
 @pytest.mark.parametrize("t,h,hkv,d,n_past", [(128, 8, 2, 128, 0), (129, 16, 4, 64, 67), (256, 4, 2, 64, 401),
-                                              (103, 10, 2, 128, 1001)])
+                                              (103, 10, 2, 128, 1001), (257, 4, 1, 128, 1793)])
 def test_many_rows_take_limb_caches(ctx, t, h, hkv, d, n_past):
     # 512 and more query rows per KV head: the caches are made into limbs
     # first; n = 128, 196, 657, 1104 rows (strides that are and are not whole
-    # 16-row segments), and 515 rows, a last block of 3
+    # 16-row segments), 515 query rows, a last block of 3; 1028 over 17
+    # chunks, in blocks of 48
     close(*run(ctx, t, h, hkv, d, n_past, None, extra_rows=3))
 
 
