@@ -51,8 +51,11 @@ constexpr int VLIMBS = CPV_ATTN_VLIMBS;
 constexpr int QB_CHAIN = 32;        // query rows per chunk workgroup: chains, prefill, fewer than 512 units;
 constexpr int QB_WIDE = 48;         //   from 512 (chunk, KV head) units on, when a KV head has more than 32,
 constexpr int QB_TREE = 80;         //   or, over the API's caches, 49 to 80 (a 16-node tree's 5 x 16)
-constexpr int64_t LIMB_ROWS = 512;  // query rows per KV head from which the API's caches become limb caches first
-constexpr size_t LIMB_BYTES = (size_t)256 << 20;   //   and the most those may take
+constexpr int64_t LIMB_ROWS = 512;  // query rows per KV head from which the API's caches become limb caches first,
+constexpr size_t LIMB_BYTES = (size_t)256 << 20;   //   and the most those may take; the same where the f16 form
+constexpr int64_t LIMB_ROWS_WIDE = 1536;           //   runs in 48-row blocks at d = 128, and the most
+constexpr size_t LIMB_BYTES_WIDE = (size_t)112 << 20, LIMB_BYTES_ROW = 52 << 10;   //   at all and per query row
+constexpr int64_t WIDE_UNITS = 512; // (chunk, KV head) units from which query blocks are wide
 constexpr int E_EMPTY = CPV_E_EMPTY;   // exponent of an all-zero vector
 
 __device__ __forceinline__ int ceil_log2_dev(int64_t v)
@@ -793,7 +796,7 @@ cpv_status attn_block(cpv_ctx* ctx, const float* q, const uint16_t* kc, const ui
     // us, 24/4: 268 -> 258; after 1000, 9 to 12 chunks, no gain; at d = 64
     // 32/4: 222 -> 233).
     const bool many = D == 128 && vl && LR >= 1024 && nchunk >= 16;
-    const bool wide = many || (LR > QB_CHAIN && (int64_t)nchunk * Hkv >= 512);
+    const bool wide = many || (LR > QB_CHAIN && (int64_t)nchunk * Hkv >= WIDE_UNITS);
     const bool tree_blk = wide && !vl && LR > QB_WIDE && LR <= QB_TREE;
     const int QB = tree_blk ? QB_TREE : wide ? QB_WIDE : QB_CHAIN;
     const dim3 cgrid((unsigned)(nchunk * Hkv), 1u, (unsigned)((LR + QB - 1) / QB));
@@ -834,6 +837,36 @@ bool attn_one_block(int64_t n_past, int t, int h)
     return ((int64_t)192 << 20) / (per_token + 1) >= t;
 }
 
+// the limb caches' row stride and bytes: K's, rounded up to 256, then V's
+int64_t limb_stride(int64_t n) { return (n + 15) & ~(int64_t)15; }
+size_t k_limb_bytes(int64_t n, int h_kv, int d)
+{
+    return ((size_t)cpv_k_cache_bytes(h_kv, d, limb_stride(n)) + 255) & ~(size_t)255;
+}
+size_t limb_bytes(int64_t n, int h_kv, int d)
+{
+    return k_limb_bytes(n, h_kv, d) + (size_t)h_kv * d * limb_stride(n) * VLIMBS;
+}
+
+// Whether a chain's call over the API's caches makes them into limb caches
+// first.  Each block of query rows else converts every chunk's K and V again;
+// the conversion costs a launch and the limbs 1.5 times the bytes.  Where the
+// f16 form runs in 32-row blocks that pays from 512 rows per KV head on (40/8
+// x 128, 3584 rows before: 640 rows 122.6 -> 119.1 us, 2560 rows 481 -> 418;
+// 320 rows 67.9 -> 67.8), and at d = 64 over 48-row blocks too (32/4, 16384
+// rows: 640 rows 169 -> 166).  At d = 128 over 48-row blocks (fewer
+// conversions to save) it pays while the limbs stay in the 256 MB behind the
+// L2s beside the partials (40/8: 512 to 1024 rows 1.0 to 1.06 times the f16
+// form's time; 1536 rows over 75 MB 0.974, over 101 MB 1.02; 2048 over 103 MB
+// 0.992, over 122 MB 1.012; 2560 over 200 MB 1.02).
+bool limbs_pay(int64_t n, int64_t rows, int h_kv, int d)
+{
+    const bool wide = d == 128 && (n + CHUNK - 1) / CHUNK * h_kv >= WIDE_UNITS;
+    const size_t bytes = limb_bytes(n, h_kv, d);
+    if (!wide) return rows >= LIMB_ROWS && bytes <= LIMB_BYTES;
+    return rows >= LIMB_ROWS_WIDE && bytes <= LIMB_BYTES_WIDE && bytes <= (size_t)rows * LIMB_BYTES_ROW;
+}
+
 template <int D>
 cpv_status attn_run(cpv_ctx* ctx, const float* q, const uint16_t* kc, const uint16_t* vt, int64_t v_stride,
                     int64_t n_past, const int32_t* parent, int t, int h, int h_kv, float scale, float* out,
@@ -849,21 +882,14 @@ cpv_status attn_run(cpv_ctx* ctx, const float* q, const uint16_t* kc, const uint
     int64_t tb = ((int64_t)192 << 20) / (per_token + 1);
     if (tb < 1) tb = 1;
     if (tb > t) tb = t;
-    // The API's caches under many query rows: made into limb caches first.
-    // Each block of 32 rows else converts every chunk's K and V again; from
-    // 512 rows per KV head the conversion's launch and the limbs' 1.5 times
-    // the bytes cost less (40/8 x 128, 3584 rows before: 640 rows 120 -> 113
-    // us, 2560 rows 480 -> 430; 320 rows 67.9 -> 67.8, and over 16384 rows
-    // 226 -> 252).
-    const int64_t ls = (n + 15) & ~(int64_t)15;
-    const size_t kl_b = ((size_t)cpv_k_cache_bytes(h_kv, D, ls) + 255) & ~(size_t)255;
-    const size_t vl_b = (size_t)h_kv * D * ls * VLIMBS;
+    // the API's caches under many query rows: made into limb caches first
     size_t off = 0;
-    if (!vl && (int64_t)(h / h_kv) * t >= LIMB_ROWS && kl_b + vl_b <= LIMB_BYTES) {
+    if (!vl && limbs_pay(n, (int64_t)(h / h_kv) * t, h_kv, D)) {
         // all of the call's workspace at once: growth would drop the caches
-        const int64_t rows = tb * h, nc = (n + CHUNK - 1) / CHUNK;
+        const int64_t rows = tb * h, nc = (n + CHUNK - 1) / CHUNK, ls = limb_stride(n);
+        const size_t kl_b = k_limb_bytes(n, h_kv, D), kv_b = limb_bytes(n, h_kv, D);
         void* ws = nullptr;
-        cpv_status st = cpv_workspace(ctx, kl_b + vl_b + (size_t)nc * rows * (D * 4 + 12) + 3 * 256, &ws);
+        cpv_status st = cpv_workspace(ctx, kv_b + (size_t)nc * rows * (D * 4 + 12) + 3 * 256, &ws);
         if (st != CPV_OK) return st;
         const int64_t kb = (n * h_kv * (D / 16) + 255) / 256, vb = ((int64_t)h_kv * D * (ls / 16) + 255) / 256;
         kv_limbs_kernel<D><<<(unsigned)(kb + vb), 256, 0, ctx->stream>>>(kc, vt, v_stride, n, ls, h_kv, (int8_t*)ws,
@@ -872,7 +898,7 @@ cpv_status attn_run(cpv_ctx* ctx, const float* q, const uint16_t* kc, const uint
         kl = (int8_t*)ws;
         vl = (int8_t*)ws + kl_b;
         v_stride = ls;
-        off = kl_b + vl_b;
+        off = kv_b;
     }
     for (int t0 = 0; t0 < t; t0 += (int)tb) {
         const int tn = t - t0 < (int)tb ? t - t0 : (int)tb;
@@ -930,6 +956,11 @@ cpv_status cpv_attn_partials(cpv_ctx* ctx, const float* q, const uint16_t* kc, c
         cpv_prof_keep(ctx, CPV_PROF_ATTN, bytes, [go]() { (void)go(true); });
     }
     return st;
+}
+
+extern "C" int cpv_attn_takes_limbs(int64_t n_past, int t, int h, int h_kv, int d)
+{
+    return limbs_pay(n_past + t, (int64_t)(h / h_kv) * t, h_kv, d) ? 1 : 0;
 }
 
 extern "C" cpv_status cpv_attn(cpv_ctx* ctx, const float* q_dev, const uint16_t* k_cache_dev,

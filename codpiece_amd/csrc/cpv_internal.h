@@ -514,6 +514,9 @@ __device__ __forceinline__ void cpv_k_limbs(float kf, int e, int8_t* hi, int8_t*
 cpv_status cpv_attn_launch(cpv_ctx* ctx, const float* q, const uint16_t* kc, const uint16_t* vt, int64_t v_stride,
                            int64_t n_past, const int32_t* parent, int t, int h, int h_kv, int d, float scale,
                            float* out, const int8_t* vl = nullptr, const int8_t* kl = nullptr);
+// what a chain's dispatch over the API's caches picks: 1 where they become
+// limb caches first (a host query, for the tests)
+extern "C" int cpv_attn_takes_limbs(int64_t n_past, int t, int h, int h_kv, int d);
 cpv_status cpv_qgemm_launch(cpv_ctx* ctx, const cpv_weight* w, const float* x, int64_t m, float* y);
 
 // the attention's chunk partials for a consumer that folds them itself (chains
