@@ -882,23 +882,31 @@ cpv_status attn_run(cpv_ctx* ctx, const float* q, const uint16_t* kc, const uint
     int64_t tb = ((int64_t)192 << 20) / (per_token + 1);
     if (tb < 1) tb = 1;
     if (tb > t) tb = t;
-    // the API's caches under many query rows: made into limb caches first
+    // the API's caches under many query rows: made into limb caches first,
+    // where the workspace has the room or may grow to it (else as they are: a
+    // call that is being captured, or that fills the device, runs all the same)
     size_t off = 0;
     if (!vl && limbs_pay(n, (int64_t)(h / h_kv) * t, h_kv, D)) {
         // all of the call's workspace at once: growth would drop the caches
         const int64_t rows = tb * h, nc = (n + CHUNK - 1) / CHUNK, ls = limb_stride(n);
         const size_t kl_b = k_limb_bytes(n, h_kv, D), kv_b = limb_bytes(n, h_kv, D);
+        const size_t need = kv_b + (size_t)nc * rows * (D * 4 + 12) + 3 * 256;
         void* ws = nullptr;
-        cpv_status st = cpv_workspace(ctx, kv_b + (size_t)nc * rows * (D * 4 + 12) + 3 * 256, &ws);
-        if (st != CPV_OK) return st;
-        const int64_t kb = (n * h_kv * (D / 16) + 255) / 256, vb = ((int64_t)h_kv * D * (ls / 16) + 255) / 256;
-        kv_limbs_kernel<D><<<(unsigned)(kb + vb), 256, 0, ctx->stream>>>(kc, vt, v_stride, n, ls, h_kv, (int8_t*)ws,
-                                                                        (int8_t*)ws + kl_b, (int)kb);
-        CPV_HIP(ctx, hipGetLastError());
-        kl = (int8_t*)ws;
-        vl = (int8_t*)ws + kl_b;
-        v_stride = ls;
-        off = kv_b;
+        if (need <= ctx->ws_bytes || !cpv_capturing(ctx)) {
+            cpv_status st = cpv_workspace(ctx, need, &ws);
+            if (st == CPV_ENOMEM) ws = nullptr;
+            else if (st != CPV_OK) return st;
+        }
+        if (ws) {
+            const int64_t kb = (n * h_kv * (D / 16) + 255) / 256, vb = ((int64_t)h_kv * D * (ls / 16) + 255) / 256;
+            kv_limbs_kernel<D><<<(unsigned)(kb + vb), 256, 0, ctx->stream>>>(kc, vt, v_stride, n, ls, h_kv, (int8_t*)ws,
+                                                                            (int8_t*)ws + kl_b, (int)kb);
+            CPV_HIP(ctx, hipGetLastError());
+            kl = (int8_t*)ws;
+            vl = (int8_t*)ws + kl_b;
+            v_stride = ls;
+            off = kv_b;
+        }
     }
     for (int t0 = 0; t0 < t; t0 += (int)tb) {
         const int tn = t - t0 < (int)tb ? t - t0 : (int)tb;

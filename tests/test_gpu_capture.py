@@ -72,3 +72,39 @@ def test_buffer_growth_is_refused_inside_a_capture():
     w1.free()
     w2.free()
     ctx.close()
+
+
+def test_a_prompt_chunk_is_captured_in_the_workspace_of_another():
+    # 512 query rows per KV head make the caches into limb caches where the
+    # workspace has the room; in a capture after a call that left less (but
+    # enough without them) the chunk runs on the caches as they are
+    from codpiece_amd.runtime import Context
+    ctx = Context(0)
+    rng = np.random.default_rng(6)
+    h, hkv, d, t, n_past = 8, 2, 128, 128, 4000
+    n_max, vs = 4736, 4736
+    k = cpvo.f32_to_f16_bits(rng.normal(size=(n_max, hkv * d)).astype(np.float32))
+    v = cpvo.f32_to_f16_bits(rng.normal(size=(n_max, hkv * d)).astype(np.float32))
+    kt, vt = (torch.from_numpy(np.ascontiguousarray(x).view(np.int16)).cuda() for x in (k, v.T))
+    q = rng.normal(size=(t, h, d)).astype(np.float32)
+    qt = torch.from_numpy(q).cuda()
+    out = torch.zeros((t, h * d), device="cuda")
+    scale = np.float32(1) / np.sqrt(np.float32(d))
+    # 480 rows per KV head over 37 chunks: more partials than the chunk has, no limb caches
+    ctx.attn(qt[:120], kt, vt, 4600, None, hkv, float(scale))
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ctx.use_stream(torch.cuda.current_stream())
+        ctx.attn(qt, kt, vt, n_past, None, hkv, float(scale), out=out)
+    ctx.use_stream(torch.cuda.current_stream())
+    ref = cpvo.attn(q, k[:n_past + t], v[:n_past + t], n_past, None, scale)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        assert np.array_equal(out.cpu().numpy(), ref)
+    # eagerly the workspace grows and the limb caches give the same (the graph
+    # holds the old workspace: it goes first)
+    del graph
+    assert np.array_equal(ctx.attn(qt, kt, vt, n_past, None, hkv, float(scale)).cpu().numpy(), ref)
+    ctx.close()
