@@ -309,6 +309,10 @@ cpv_status cpv_qgemm_act(cpv_ctx* ctx, const cpv_weight* w, const cpv_act* act, 
 // Q8_0 (cpv_qgemm_wide_ok).
 bool cpv_qgemm_wide_ok(const cpv_weight* w, int64_t m);
 cpv_status cpv_qgemm_wide(cpv_ctx* ctx, const cpv_weight* w, const cpv_act* act, double* gsum, int win, float* y);
+// what they pick for m rows against [n][k] on cus CUs: 16-row blocks per
+// workgroup, row blocks, (tile, row block) pairs over all of K, K slices of
+// the others, units a slice; 0 where they refuse (a host query, for the tests)
+extern "C" int cpv_qgemm_wide_plan(int type, int64_t n, int64_t k, int64_t m, int cus, int out[5]);
 
 // A GEMM result kept in the accumulator for a fused consumer: row m, output n
 // is cpv_gout_value(acc[m * n_pad + n], ew[n], Ea(m), win) with Ea(m) the

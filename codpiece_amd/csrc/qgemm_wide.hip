@@ -677,19 +677,26 @@ namespace {
 // pairs 55; 5120 x 17408 at 256 rows: 8 blocks in 160 pairs x 3 slices 112, 4
 // in 320 whole pairs 146; Q8_0 7168 x 5120 at 201 rows: 3 blocks in 560 pairs
 // 75, 2 in 784 pairs 63.
-void wide_split(WideArgs& a, bool q80, int maxb, int cus, int* nmt_out)
+// Returns false where no deal's workgroups fit a grid.
+struct WidePlan { int nmt, mblocks, nfull, ksplit, upk; };
+
+bool wide_plan(bool q80, int64_t tiles, int M, int U, int cus, WidePlan* p)
 {
-    const int nb16 = (a.M + 15) / 16;
+    // (the staging offsets within a row block are 32-bit: very long rows in smaller blocks)
+    int maxb = q80 ? MAX_NMT_Q80 : MAX_NMT;
+    while (16LL * maxb * U * 256 > INT32_MAX) maxb--;
+    const int nb16 = (M + 15) / 16;
     double best = 1e30;
     for (int mb = (nb16 + maxb - 1) / maxb; mb <= nb16; mb++) {
         const int nmt = (nb16 + mb - 1) / mb;
         if ((nb16 + nmt - 1) / nmt != mb) continue;   // (the same blocks in fewer workgroups)
         const int slots = cus * wide_per_cu(q80, nmt);
-        const int64_t pairs = (int64_t)a.tiles * mb, full = pairs / slots * slots, rest = pairs - full;
+        const int64_t pairs = tiles * mb, full = pairs / slots * slots, rest = pairs - full;
+        if (full + 16LL * slots > (int64_t)(UINT32_MAX / WT)) break;
         const double t = q80 ? 0.95 * nmt : (0.5 + 0.315 * nmt) * wide_per_cu(q80, nmt) / 2, t1 = 0.62 * t, s0 = 3.0;
-        const double tf = (double)(full / slots) * (a.U * t + s0);
-        for (int ks = 1; ks == 1 || (rest && ks <= a.U / 4 && ks <= 16); ks++) {
-            const int upk = (a.U + ks - 1) / ks, k2 = (a.U + upk - 1) / upk;
+        const double tf = (double)(full / slots) * (U * t + s0);
+        for (int ks = 1; ks == 1 || (rest && ks <= U / 4 && ks <= 16); ks++) {
+            const int upk = (U + ks - 1) / ks, k2 = (U + upk - 1) / upk;
             if (k2 != ks) continue;
             const int64_t w = rest * ks, last = w % slots;
             double tr = (double)(w / slots) * (upk * t + s0);
@@ -697,15 +704,12 @@ void wide_split(WideArgs& a, bool q80, int maxb, int cus, int* nmt_out)
             if (ks > 1) tr += (double)w * nmt * 1024 * 3.5e-6 + 1.5;
             if (tf + tr < best) {
                 best = tf + tr;
-                *nmt_out = nmt;
-                a.mblocks = mb;
-                a.nfull = (int)(ks > 1 ? full : pairs);
-                a.ksplit = ks;
-                a.upk = upk;
+                *p = {nmt, mb, (int)(ks > 1 ? full : pairs), ks, upk};
             }
         }
         if (nmt <= 2) break;
     }
+    return best < 1e30;
 }
 
 void q80_launch(const WideArgs& a, int nmt, unsigned grid, hipStream_t stream)
@@ -738,13 +742,10 @@ void kq_launch(const WideArgs& a, int nmt, unsigned grid, hipStream_t stream)
 cpv_status cpv_qgemm_wide(cpv_ctx* ctx, const cpv_weight* w, const cpv_act* act, double* gsum, int win, float* y)
 {
     const bool q80 = w->type == CPV_Q8_0, q6k = w->type == CPV_Q6_K;
-    if ((w->type != CPV_Q4_K && !q80 && !q6k) || act->kq == q80 || act->U != (int)w->units || act->m < 1 ||
-        act->m > INT32_MAX / 2)
+    if ((w->type != CPV_Q4_K && !q80 && !q6k) || act->kq == q80 || act->U != (int)w->units ||
+        !cpv_qgemm_wide_ok(w, act->m) || act->m > INT32_MAX / 2)
         return cpv_fail(ctx, CPV_EINVAL, "qgemm_wide: weight or activation format not supported");
-    // (the staging offsets within a row block are 32-bit: very long rows in smaller blocks)
-    int maxb = q80 ? MAX_NMT_Q80 : MAX_NMT;
-    while (maxb > 0 && 16LL * maxb * act->U * 256 > INT32_MAX) maxb--;
-    if (maxb == 0)
+    if (64LL * act->U * 256 > INT32_MAX)
         return cpv_fail(ctx, CPV_EUNSUPPORTED, "qgemm_wide: k=%lld too long", (long long)w->k);
     WideArgs a;
     a.w = (const uint8_t*)w->data;
@@ -762,10 +763,14 @@ cpv_status cpv_qgemm_wide(cpv_ctx* ctx, const cpv_weight* w, const cpv_act* act,
     a.y = y;
     a.n = w->n;
     a.vec = (w->n & 3) == 0 && ((uintptr_t)y & 15) == 0;
-    if ((int64_t)a.tiles * ((a.M + 15) / 16) > INT32_MAX / 1024)
+    WidePlan p;
+    if (!wide_plan(q80, a.tiles, a.M, a.U, ctx->cu_count, &p))
         return cpv_fail(ctx, CPV_EUNSUPPORTED, "qgemm_wide: %d tiles by %d rows", a.tiles, a.M);
-    int nmt = 4;
-    wide_split(a, q80, maxb, ctx->cu_count, &nmt);
+    const int nmt = p.nmt;
+    a.mblocks = p.mblocks;
+    a.nfull = p.nfull;
+    a.ksplit = p.ksplit;
+    a.upk = p.upk;
     const int64_t blocks = (int64_t)a.tiles * a.mblocks;
     const int64_t rest = blocks - a.nfull, grid = a.nfull + rest * a.ksplit;
     const int ev = cpv_prof_mark(ctx);
@@ -787,4 +792,19 @@ cpv_status cpv_qgemm_wide(cpv_ctx* ctx, const cpv_weight* w, const cpv_act* act,
         cpv_prof_keep(ctx, cls, bytes, go);
     }
     return CPV_OK;
+}
+
+extern "C" int cpv_qgemm_wide_plan(int type, int64_t n, int64_t k, int64_t m, int cus, int out[5])
+{
+    WidePlan p{};
+    const int64_t U = (k + 255) / 256;
+    if (m < 1 || m > INT32_MAX / 2 || 64 * U * 256 > INT32_MAX ||
+        !wide_plan(type == CPV_Q8_0, (n + 63) / 64, (int)m, (int)U, cus, &p))
+        return 0;
+    out[0] = p.nmt;
+    out[1] = p.mblocks;
+    out[2] = p.nfull;
+    out[3] = p.ksplit;
+    out[4] = p.upk;
+    return 1;
 }

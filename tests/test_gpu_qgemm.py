@@ -149,6 +149,28 @@ def test_qgemm_wide_whole_and_sliced(ctx, tname):
         assert np.array_equal(y.view(np.uint32), ref.view(np.uint32)), np.abs(y - ref).max()
 
 
+def test_qgemm_wide_many_weight_rows():
+    # 131,100 tiles by 16 row blocks: the first, a middle and the last weight
+    # rows against the same rows on their own (a context of its own: 17 GB of
+    # accumulator)
+    from codpiece_amd.runtime import Context
+    ctx = Context(0)
+    n, k, m = 64 * 131099 + 7, 32, 256
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    raw = torch.randint(0, 256, (n, 34), dtype=torch.uint8, device="cuda", generator=gen)
+    raw[:, :2] = (0.001 + 0.01 * torch.rand(n, 1, device="cuda", generator=gen)).half().view(torch.uint8)
+    x = torch.randn(m, k, device="cuda", generator=gen)
+    w = ctx.upload_weight(cpvo.Q8_0, raw.view(-1), n, k)
+    print(f"case n={n} k={k} m={m}", flush=True)
+    y = ctx.qgemm(w, x)
+    w.free()
+    for r0 in (0, 4_000_003, n - 1000):
+        part = ctx.upload_weight(cpvo.Q8_0, raw[r0:r0 + 1000].reshape(-1).contiguous(), 1000, k)
+        assert torch.equal(y[:, r0:r0 + 1000], ctx.qgemm(part, x))
+        part.free()
+    ctx.close()
+
+
 @pytest.mark.parametrize("m", [32, 100])
 def test_qgemm_wide_q8_0_partial_unit(ctx, m):
     # K = 800: 25 blocks of 32, so the last 256-element unit holds one block
