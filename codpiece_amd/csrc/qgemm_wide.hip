@@ -41,13 +41,13 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef unsigned short v2u __attribute__((ext_vector_type(2)));
 
 struct WideArgs {
-    const uint8_t* w;      // repacked Q4_K tiles: [tile][unit][9 pieces][64 rows][16 B]
+    const uint8_t* w;      // repacked tiles: [tile][unit][pieces: Q4_K 9, Q6_K 13, Q8_0 17][64 rows][16 B]
     const int32_t* ew;     // [n_pad] row exponents
     const int8_t* qa;      // [rows][U*256] activation codes
     const float* da;       // [rows][U] activation scales
     double* gsum;          // [rows][n_pad], zero on entry
     int64_t n_pad;
-    int U, M, m0, win;
+    int U, M, win;
     int tiles, mblocks, ksplit, upk;   // grid = tiles * mblocks * ksplit; upk units per K slice
     const int32_t* bs16;   // [rows][U*16] sums of 16 codes (Q8_K)
     float* y;              // outputs [rows][n], or null: the sums stay in gsum
@@ -726,7 +726,9 @@ template <int TYPE>
 void kq_launch(const WideArgs& a, int nmt, unsigned grid, hipStream_t stream)
 {
     switch (nmt) {
-    case 1: qgemm_wide_kq_kernel<TYPE, 1><<<grid, WT, 0, stream>>>(a); break;
+    case 1:   // (9 to 16 rows: Q6_K only)
+        if constexpr (TYPE == CPV_Q6_K) qgemm_wide_kq_kernel<TYPE, 1><<<grid, WT, 0, stream>>>(a);
+        break;
     case 2: qgemm_wide_kq_kernel<TYPE, 2><<<grid, WT, 0, stream>>>(a); break;
     case 3: qgemm_wide_kq_kernel<TYPE, 3><<<grid, WT, 0, stream>>>(a); break;
     case 4: qgemm_wide_kq_kernel<TYPE, 4><<<grid, WT, 0, stream>>>(a); break;
@@ -756,7 +758,6 @@ cpv_status cpv_qgemm_wide(cpv_ctx* ctx, const cpv_weight* w, const cpv_act* act,
     a.n_pad = w->n_pad;
     a.U = act->U;
     a.M = (int)act->m;
-    a.m0 = 0;
     a.win = win;
     a.tiles = (int)(w->n_pad / 64);
     a.bs16 = act->bs16;
