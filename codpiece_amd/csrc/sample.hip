@@ -44,7 +44,7 @@ constexpr int BU = 8;                  // strided loops: loads issued ahead of t
 constexpr uint32_t FTOP = 1u << 24;    // fold: ulps from 0 to the top of a binade
 constexpr uint32_t FSAT = 1u << 26;    // fold: saturation of a composed step
 constexpr int FOLD_SEQ = 1024;         // folds: leading elements added by one thread
-constexpr int BAND = 16384;            // sorted band held in LDS as u64 keys
+constexpr int LBAND = 14, BAND = 1 << LBAND;   // sorted band held in LDS as u64 keys
 constexpr int HIST_MAX = 4096;         // penalty window input limit (4 per thread)
 constexpr int VMAX = 262144;           // ids fit the low 18 bits of a key
 // a band in candidate order: a block radix sort of 16 keys per thread, each
@@ -649,8 +649,9 @@ __device__ __forceinline__ void sort_emit(const float* lg, int cnt, int pos, int
 
 // the split top-p build's state per row: the row maximum in EXP_SPLIT
 // parts, then what its first launch leaves for the second
-constexpr int EXP_SPLIT = 32;
-constexpr int FCAP = BAND / EXP_SPLIT;   // keys a part may select for a top-k or min-p build
+constexpr int EXP_SPLIT = 32, LNP_MAX = 5;
+static_assert(EXP_SPLIT == 1 << LNP_MAX, "log2 of the most parts");
+constexpr int PART_MAX = 8192;           // most elements of a part of the part kernels (2^lnp parts, DistArgs)
 constexpr int FRONT_K = 256;             // top-k counts up to this select by parts
 constexpr int FT = 512;                  // threads of the part kernels (four workgroups share a CU)
 struct DistState {
@@ -666,7 +667,7 @@ struct DistState {
     unsigned long long first;   // the band's first key
     float bf1[MAXP], bf2[MAXP]; // each part's estimated sums of exp(l - max) and exp((l - max) / T)
     // top-k and min-p builds (front_kernel, floor_kernel): each part's number
-    // of selected keys (kept in bkeys, FCAP a part), and the histogram bin
+    // of selected keys (kept in bkeys, BAND >> lnp a part), and the histogram bin
     // they reach (top-k) or the number of logits at or above the floor (min-p)
     int fcnt[EXP_SPLIT], fval[EXP_SPLIT];
     int wn;                     // penalties: the window's distinct tokens (window_kernel)
@@ -920,6 +921,7 @@ struct DistArgs {
     unsigned long long* bkeys;  // [rows][BAND] the first band's keys, part by part (phase 1)
     float* e2;                  // [rows][BAND] exp(l / T - mx2) of the first band's candidates (band parts)
     int sel;                    // the candidates come from front_kernel (top-k: the count) or floor_kernel (min-p: -1)
+    int lnp;                    // log2 of the parts per row of front_kernel and floor_kernel
     int parts;                  // phase 1 leaves the first band in parts (band_part_kernel follows)
 };
 
@@ -1008,9 +1010,9 @@ __device__ __forceinline__ const float* row_logits(const DistArgs& a, int row)
 // the row maximum in parts (fmaxf is order-free), then pr[i] = expf(l - max)
 // by index, as the one-workgroup build computes them.
 // the part's element range, in whole float4s (parts start at multiples of 4)
-__device__ __forceinline__ void exp_part(int V, int part, int* i0, int* i1)
+__device__ __forceinline__ void exp_part(int V, int part, int* i0, int* i1, int lnp = LNP_MAX)
 {
-    const int per = (((V + EXP_SPLIT - 1) / EXP_SPLIT) + 3) & ~3;
+    const int per = (((V + (1 << lnp) - 1) >> lnp) + 3) & ~3;
     *i0 = min(V, part * per);
     *i1 = min(V, *i0 + per);
 }
@@ -1106,16 +1108,17 @@ __global__ __launch_bounds__(256) void fmap_kernel(DistArgs a)
     }
 }
 
-// What a build needs of the whole row before its candidates, EXP_SPLIT
-// workgroups per row (one workgroup streams a row at 60-100 GB/s, 6-10 us a
-// pass over 151,936 logits, and took five passes): the penalised copy and the
+// What a build needs of the whole row before its candidates, 2^lnp workgroups
+// per row (one workgroup streams a row at 60-100 GB/s, 6-10 us a pass over
+// 151,936 logits, and took five passes): the penalised copy and the
 // part's maximum, and for a top-k build (sel > 0) the part's keys down to its
 // sel-th largest.  Those are whole bins of a histogram over the keys' top 12
 // bits: the row's sel largest keys lie in the bins up to the smallest such
 // bin of any part (the part that has it holds sel keys there), and every part
 // has given all its keys in those.
-constexpr int PART_MAX = (VMAX / EXP_SPLIT + 3) & ~3, PIPT = (PART_MAX + FT - 1) / FT;
-// the part's elements of this thread, i0 + tid + q SB (loads issued together, at clamped indices)
+constexpr int PIPT = PART_MAX / FT;
+static_assert(PART_MAX * EXP_SPLIT >= VMAX && PART_MAX % FT == 0, "a row's parts hold it");
+// the part's elements of this thread, i0 + tid + q FT (loads issued together, at clamped indices)
 __device__ __forceinline__ void part_load(const float* lg, int i0, int i1, float (&v)[PIPT])
 {
 #pragma unroll
@@ -1132,8 +1135,14 @@ __global__ __launch_bounds__(FT) void front_kernel(DistArgs a)
     __shared__ Small sm;
     const int part = blockIdx.y, row = blockIdx.x, V = a.V, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     DistState& st = a.st[row];
+    // (entries that have no part, for the readers of all EXP_SPLIT)
+    for (int q = tid + (1 << a.lnp); part == 0 && q < EXP_SPLIT; q += FT) {
+        st.pmax[q] = -INFINITY;
+        st.fcnt[q] = 0;
+        st.fval[q] = a.sel < 0 ? 0 : 4095;
+    }
     int i0, i1;
-    exp_part(V, part, &i0, &i1);
+    exp_part(V, part, &i0, &i1, a.lnp);
     const int n = i1 - i0;
     if (n <= 0) {                              // (the whole workgroup)
         if (tid == 0) {
@@ -1204,12 +1213,13 @@ __global__ __launch_bounds__(FT) void front_kernel(DistArgs a)
     }
     __syncthreads();
     const uint32_t bin = (uint32_t)sm.iv[0];
-    unsigned long long* out = a.bkeys + (size_t)row * BAND + part * FCAP;
+    const int cap = BAND >> a.lnp;
+    unsigned long long* out = a.bkeys + (size_t)row * BAND + part * cap;
 #pragma unroll
     for (int q = 0; q < PIPT; q++)
         if (tid + q * FT < n && desc_key(v[q]) >> 20 <= bin) {
             const int at = atomicAdd(&sm.iv[1], 1);
-            if (at < FCAP) out[at] = cand_key(v[q], i0 + tid + q * FT);
+            if (at < cap) out[at] = cand_key(v[q], i0 + tid + q * FT);
         }
     __syncthreads();
     if (tid == 0) {
@@ -1234,7 +1244,7 @@ __global__ __launch_bounds__(FT) void floor_kernel(DistArgs a)
     const int part = blockIdx.y, row = blockIdx.x, V = a.V, tid = threadIdx.x;
     DistState& st = a.st[row];
     int i0, i1;
-    exp_part(V, part, &i0, &i1);
+    exp_part(V, part, &i0, &i1, a.lnp);
     if (i0 >= i1) {                            // (the whole workgroup)
         if (tid == 0) st.fcnt[part] = st.fval[part] = 0;
         return;
@@ -1245,7 +1255,8 @@ __global__ __launch_bounds__(FT) void floor_kernel(DistArgs a)
     const uint32_t fk = desc_key(floor_l);
     if (tid < 2) s_n[tid] = 0;
     __syncthreads();
-    unsigned long long* out = a.bkeys + (size_t)row * BAND + part * FCAP;
+    const int cap = BAND >> a.lnp;
+    unsigned long long* out = a.bkeys + (size_t)row * BAND + part * cap;
     int cnt = 0;
 #pragma unroll
     for (int q = 0; q < PIPT; q++) {
@@ -1254,7 +1265,7 @@ __global__ __launch_bounds__(FT) void floor_kernel(DistArgs a)
         cnt += v[q] >= floor_l ? 1 : 0;
         if (desc_key(v[q]) <= fk) {
             const int at = atomicAdd(&s_n[0], 1);
-            if (at < FCAP) out[at] = cand_key(v[q], i);
+            if (at < cap) out[at] = cand_key(v[q], i);
         }
     }
     cnt = cpv_wave_reduce(cnt, cpv_op_add());
@@ -1272,35 +1283,32 @@ __global__ __launch_bounds__(FT) void floor_kernel(DistArgs a)
 // told from more than a key per thread (the caller then emits bands).  The
 // keys with the M largest logits lie in the first bins of a histogram over
 // the selected keys' own range of desc_key (4096 bins).
+template <bool MOST>   // EXP_SPLIT parts (a fixed layout of the keys: 0.3 us)
 __device__ __noinline__ int emit_selected(const float* lg, const DistState* stp, const unsigned long long* src,
-                                          bool bins, int M, int32_t* sid, float* sl, unsigned long long* keys,
+                                          int lnp, bool bins, int M, int32_t* sid, float* sl, unsigned long long* keys,
                                           Small* sm)
 {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const DistState& st = *stp;
     const int fc = lane < EXP_SPLIT ? st.fcnt[lane] : 0, fv = lane < EXP_SPLIT ? st.fval[lane] : 4095;
-    if (M < 1 || __builtin_amdgcn_ballot_w64(fc > FCAP)) return 0;   // (the same in every wave)
-    // a wave takes part wave, then part wave + SWV
-    constexpr int KPL = FCAP / 64, PPW = EXP_SPLIT / SWV;
-    static_assert(PPW * SWV == EXP_SPLIT && KPL * 64 == FCAP, "whole parts per wave");
+    const int lcap = LBAND - (MOST ? LNP_MAX : lnp), cap = 1 << lcap;
+    if (M < 1 || __builtin_amdgcn_ballot_w64(fc > cap)) return 0;   // (the same in every wave)
+    constexpr int KPT = BAND / SB;
+    static_assert(BAND / EXP_SPLIT % 64 == 0, "a wave's 64 slots lie in one part");
     // (top-k: every part's keys are complete down to the smallest bin only)
     const int bin = bins ? (int)-cpv_wave_reduce(-(float)fv, cpv_op_max()) : 4095;
-    unsigned long long k[PPW][KPL];
+    unsigned long long k[KPT];
     uint32_t lo = ~0u, hi = 0u;
 #pragma unroll
-    for (int p = 0; p < PPW; p++) {
-        const int part = wave + p * SWV;
-        const int n = __builtin_amdgcn_readlane(fc, __builtin_amdgcn_readfirstlane(part));
-#pragma unroll
-        for (int q = 0; q < KPL; q++) {
-            const int i = lane + 64 * q;
-            k[p][q] = src[part * FCAP + (i < n ? i : 0)];
-            if (i >= n || (int)(k[p][q] >> 52) > bin) k[p][q] = ~0ull;
-            if (k[p][q] != ~0ull) {
-                const uint32_t d = (uint32_t)(k[p][q] >> 32);
-                lo = d < lo ? d : lo;
-                hi = d > hi ? d : hi;
-            }
+    for (int q = 0; q < KPT; q++) {
+        const int slot = (__builtin_amdgcn_readfirstlane(wave) * KPT + q) * 64, part = slot >> lcap;
+        const int n = __builtin_amdgcn_readlane(fc, part), i = (slot & (cap - 1)) + lane;
+        k[q] = src[(part << lcap) + (i < n ? i : 0)];
+        if (i >= n || (int)(k[q] >> 52) > bin) k[q] = ~0ull;
+        if (k[q] != ~0ull) {
+            const uint32_t d = (uint32_t)(k[q] >> 32);
+            lo = d < lo ? d : lo;
+            hi = d > hi ? d : hi;
         }
     }
     uint32_t* hist = (uint32_t*)(keys + SB);   // after the kept keys
@@ -1322,10 +1330,8 @@ __device__ __noinline__ int emit_selected(const float* lg, const DistState* stp,
     if (lo > hi) return 0;                     // (no key)
     const int sh = hi - lo < 4096u ? 0 : 20 - __builtin_clz(hi - lo);
 #pragma unroll
-    for (int p = 0; p < PPW; p++)
-#pragma unroll
-        for (int q = 0; q < KPL; q++)
-            if (k[p][q] != ~0ull) atomicAdd(&hist[((uint32_t)(k[p][q] >> 32) - lo) >> sh], 1u);
+    for (int q = 0; q < KPT; q++)
+        if (k[q] != ~0ull) atomicAdd(&hist[((uint32_t)(k[q] >> 32) - lo) >> sh], 1u);
     __syncthreads();
     uint32_t c[4], sum = 0, tot;
 #pragma unroll
@@ -1341,13 +1347,11 @@ __device__ __noinline__ int emit_selected(const float* lg, const DistState* stp,
     const uint32_t last = (uint32_t)sm->iv[0];
     place[tid] = 0;
 #pragma unroll
-    for (int p = 0; p < PPW; p++)
-#pragma unroll
-        for (int q = 0; q < KPL; q++)
-            if (k[p][q] != ~0ull && ((uint32_t)(k[p][q] >> 32) - lo) >> sh <= last) {
-                const int at = atomicAdd(&sm->iv[3], 1);
-                if (at < SB) keys[at] = k[p][q];
-            }
+    for (int q = 0; q < KPT; q++)
+        if (k[q] != ~0ull && ((uint32_t)(k[q] >> 32) - lo) >> sh <= last) {
+            const int at = atomicAdd(&sm->iv[3], 1);
+            if (at < SB) keys[at] = k[q];
+        }
     __syncthreads();
     // a key's place is the number of keys before it (they are distinct),
     // counted by as many threads per key as there are
@@ -1559,7 +1563,11 @@ __global__ __launch_bounds__(SB) void dist_kernel(DistArgs a)
                 if (keep <= probe) M = keep;
             }
         }
-        if (PH == 3) emitted = emit_selected(lg, a.st + row, a.bkeys + (size_t)row * BAND, a.sel > 0, M, sid, sl, keys, sm);
+        if (PH == 3) {
+            const unsigned long long* bk = a.bkeys + (size_t)row * BAND;
+            emitted = a.lnp == LNP_MAX ? emit_selected<true>(lg, a.st + row, bk, a.lnp, a.sel > 0, M, sid, sl, keys, sm)
+                                       : emit_selected<false>(lg, a.st + row, bk, a.lnp, a.sel > 0, M, sid, sl, keys, sm);
+        }
         while (emitted < M) {
             const int cnt = emit_band(lg, V, emitted > 0, &last, M - emitted, emitted, sid, sl, keys, sm);
             if (cnt <= 0) break;
@@ -1995,13 +2003,18 @@ cpv_status dist_launch(cpv_ctx* ctx, DistArgs& a, int rows)
     // and whole bins come with them (300: the bands, 107 us at 9 rows)
     const int kk = P.top_k > P.min_keep ? P.top_k : P.min_keep;
     a.sel = P.temp > 0.0f ? top_k ? (kk <= FRONT_K ? kk : 0) : P.min_p > 0.0f ? -1 : 0 : 0;
+    // Parts: a power of two of at most PART_MAX elements each, 32 while their
+    // workgroups are in flight together (four to a CU): min-p 0.05 over 240
+    // rows of 8000: 62 us with 32, 51 with 4 (one workgroup a row: 52)
+    a.lnp = LNP_MAX;
+    while (a.lnp > 0 && ((int64_t)rows << a.lnp) > 4LL * ctx->cu_count && a.V <= (PART_MAX << (a.lnp - 1))) a.lnp--;
     if (a.pen_on || a.sel) {
         if (a.pen_on) window_kernel<<<(unsigned)rows, FT, 0, ctx->stream>>>(a);
-        const size_t part_b = a.pen_on ? (size_t)(((a.V + EXP_SPLIT - 1) / EXP_SPLIT + 3) & ~3) * 4 : 0;
-        front_kernel<<<dim3((unsigned)rows, EXP_SPLIT), FT, part_b, ctx->stream>>>(a);
+        const size_t part_b = a.pen_on ? (size_t)(((a.V + (1 << a.lnp) - 1) >> a.lnp) + 3 & ~3) * 4 : 0;
+        front_kernel<<<dim3((unsigned)rows, 1u << a.lnp), FT, part_b, ctx->stream>>>(a);
     }
     if (!a.pen_on && !a.sel && a.pre_exp) rowmax_part_kernel<<<dim3(EXP_SPLIT, (unsigned)rows), 256, 0, ctx->stream>>>(a);
-    if (a.sel < 0) floor_kernel<<<dim3((unsigned)rows, EXP_SPLIT), FT, 0, ctx->stream>>>(a);
+    if (a.sel < 0) floor_kernel<<<dim3((unsigned)rows, 1u << a.lnp), FT, 0, ctx->stream>>>(a);
     if (a.pre_exp) {
         exp_kernel<<<dim3(EXP_SPLIT, (unsigned)rows), 256, 0, ctx->stream>>>(a);
         fmap_kernel<<<dim3(EXP_SPLIT, (unsigned)rows), 256, 0, ctx->stream>>>(a);

@@ -92,19 +92,31 @@ SELECT_CASES = [dict(temp=0.7, top_k=1), dict(temp=0.8, top_k=40), dict(temp=0.8
                 dict(temp=0.0, penalty_repeat=1.5)]
 
 
+def select_rows(rng, rows, v):
+    x = spiked(rng, (rows, v))
+    x[1::6] = np.round(x[1::6])                      # ties
+    x[2::6] = 0.25                                   # all equal
+    x[3::6] = np.where(rng.random(x[3::6].shape) < 0.5, -0.0, 0.0)   # equal but for the sign of zero
+    x[4::6][rng.random(x[4::6].shape) < 0.3] = -np.inf               # banned tokens
+    x[4::6, 0] = 1.0
+    x[5::6, :v // 2] -= 40.0                         # every candidate in some of the parts
+    return x, rng.integers(-1, v, size=(rows, 40)).astype(np.int32)
+
+
 @pytest.mark.parametrize("v", [2, 31, 33, 129, 4097, 20000, 262144])
 def test_distribution_selected_by_parts(ctx, v):
-    rng = np.random.default_rng(v)
-    x = spiked(rng, (6, v))
-    x[1] = np.round(x[1])                            # ties
-    x[2] = 0.25                                      # all equal
-    x[3] = np.where(rng.random(v) < 0.5, -0.0, 0.0)  # equal but for the sign of zero
-    x[4, rng.random(v) < 0.3] = -np.inf              # banned tokens
-    x[4, 0] = 1.0
-    x[5, :v // 2] -= 40.0                            # every candidate in some of the parts
-    hist = rng.integers(-1, v, size=(6, 40)).astype(np.int32)
+    x, hist = select_rows(np.random.default_rng(v), 6, v)
     for c in SELECT_CASES:
         print(f"case v={v} {c}", flush=True)
+        check_dist(ctx, x, cpvo.SamplerParams(**c), hist if "penalty_repeat" in c else None)
+
+
+@pytest.mark.parametrize("rows,v", [(40, 9000), (140, 8193), (140, 20000), (300, 501), (1030, 1200)])
+def test_distribution_selected_by_fewer_parts(ctx, rows, v):
+    # many rows: 16, 4 (by rows, by length), 2 and 1 parts a row
+    x, hist = select_rows(np.random.default_rng(rows + v), rows, v)
+    for c in SELECT_CASES:
+        print(f"case rows={rows} v={v} {c}", flush=True)
         check_dist(ctx, x, cpvo.SamplerParams(**c), hist if "penalty_repeat" in c else None)
 
 
