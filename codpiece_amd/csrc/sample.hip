@@ -754,14 +754,12 @@ __device__ BandSel band_select(const float* lg, int V, bool have_last, unsigned 
     return b;   // (not reached: the last level's bins hold one key each)
 }
 
-// the band's keys gathered into the key buffer, sorted and written out at
-// sid/sl[pos...]; *last_io advances to the band's last key
-__device__ int band_sort_emit(const float* lg, int V, bool have_last, BandSel b,
-                              unsigned long long* last_io, int pos, int32_t* sid, float* sl,
-                              unsigned long long* keys, Small* sm)
+// the band's keys gathered into the key buffer; their number
+__device__ int band_gather(const float* lg, int V, bool have_last, unsigned long long last, const BandSel& b,
+                           unsigned long long* keys, Small* sm)
 {
     const int tid = threadIdx.x;
-    const unsigned long long last = *last_io, hi = b.hi;
+    const unsigned long long hi = b.hi;
     __syncthreads();
     if (tid == 0) sm->iv[3] = 0;
     __syncthreads();
@@ -771,7 +769,14 @@ __device__ int band_sort_emit(const float* lg, int V, bool have_last, BandSel b,
         keys[atomicAdd(&sm->iv[3], 1)] = key;   // (the band is sorted below: any order)
     });
     __syncthreads();
-    const int cnt = sm->iv[3];
+    return sm->iv[3];
+}
+
+// the key buffer's cnt keys sorted and written out at sid/sl[pos...]; *last_io
+// becomes the last of them
+__device__ int band_sort_emit(const float* lg, int cnt, unsigned long long* last_io, int pos, int32_t* sid, float* sl,
+                              unsigned long long* keys, Small* sm)
+{
     if (cnt <= SMALL_BAND) sort_emit<small_sort_t, SMALL_BAND / SB>(lg, cnt, pos, sid, sl, keys, sm);
     else sort_emit<band_sort_t, BAND / SB>(lg, cnt, pos, sid, sl, keys, sm);
     *last_io = sm->last;
@@ -780,13 +785,16 @@ __device__ int band_sort_emit(const float* lg, int V, bool have_last, BandSel b,
 }
 
 // Writes ids and logits to sid/sl[pos...], advances *last and returns the
-// band size.
+// band size.  With cnt > 0 the band is the cnt keys that the key buffer holds.
 __device__ __noinline__ int emit_band(const float* lg, int V, bool have_last, unsigned long long* last_io, int want,
-                                      int pos, int32_t* sid, float* sl, unsigned long long* keys, Small* sm)
+                                      int pos, int32_t* sid, float* sl, unsigned long long* keys, Small* sm, int cnt = 0)
 {
-    const BandSel b = band_select(lg, V, have_last, *last_io, want, keys, sm);
-    if (b.tot == 0) return 0;
-    return band_sort_emit(lg, V, have_last, b, last_io, pos, sid, sl, keys, sm);
+    if (cnt == 0) {
+        const BandSel b = band_select(lg, V, have_last, *last_io, want, keys, sm);
+        if (b.tot == 0) return 0;
+        cnt = band_gather(lg, V, have_last, *last_io, b, keys, sm);
+    }
+    return band_sort_emit(lg, cnt, last_io, pos, sid, sl, keys, sm);
 }
 
 // The first band for workgroups of its own to sort (the split top-p build):
@@ -1280,7 +1288,10 @@ __global__ __launch_bounds__(FT) void floor_kernel(DistArgs a)
 // The parts' selected keys narrowed to about M, sorted and written out as the
 // first candidates (emit_band's results): their number, at least M of them;
 // or 0 when a part selected more than it may keep or the M largest cannot be
-// told from more than a key per thread (the caller then emits bands).  The
+// told from more than a key per thread (the caller then emits bands).  A min-p
+// build of more than 3/4 of a key per thread gets all its keys in the key buffer,
+// unsorted: minus their number (emit_band takes them from there; V 32000, B =
+// 1, 2700 keys: 82 us through the bands, 54 so; without the parts 73).  The
 // keys with the M largest logits lie in the first bins of a histogram over
 // the selected keys' own range of desc_key (4096 bins).
 template <bool MOST>   // EXP_SPLIT parts (a fixed layout of the keys: 0.3 us)
@@ -1310,6 +1321,17 @@ __device__ __noinline__ int emit_selected(const float* lg, const DistState* stp,
             lo = d < lo ? d : lo;
             hi = d > hi ? d : hi;
         }
+    }
+    if (!bins && M > SB * 3 / 4) {
+        uint32_t c = 0, tot;
+#pragma unroll
+        for (int q = 0; q < KPT; q++) c += k[q] != ~0ull ? 1u : 0u;
+        uint32_t at = block_excl_scan(c, sm, &tot);
+#pragma unroll
+        for (int q = 0; q < KPT; q++)
+            if (k[q] != ~0ull) keys[at++] = k[q];
+        __syncthreads();
+        return tot >= (uint32_t)M ? -(int)tot : 0;
     }
     uint32_t* hist = (uint32_t*)(keys + SB);   // after the kept keys
     int* place = (int*)hist;                   // (over the bins, once they are read)
@@ -1567,6 +1589,7 @@ __global__ __launch_bounds__(SB) void dist_kernel(DistArgs a)
             const unsigned long long* bk = a.bkeys + (size_t)row * BAND;
             emitted = a.lnp == LNP_MAX ? emit_selected<true>(lg, a.st + row, bk, a.lnp, a.sel > 0, M, sid, sl, keys, sm)
                                        : emit_selected<false>(lg, a.st + row, bk, a.lnp, a.sel > 0, M, sid, sl, keys, sm);
+            if (emitted < 0) emitted = emit_band(lg, V, false, &last, 0, 0, sid, sl, keys, sm, -emitted);
         }
         while (emitted < M) {
             const int cnt = emit_band(lg, V, emitted > 0, &last, M - emitted, emitted, sid, sl, keys, sm);
@@ -2005,7 +2028,7 @@ cpv_status dist_launch(cpv_ctx* ctx, DistArgs& a, int rows)
     a.sel = P.temp > 0.0f ? top_k ? (kk <= FRONT_K ? kk : 0) : P.min_p > 0.0f ? -1 : 0 : 0;
     // Parts: a power of two of at most PART_MAX elements each, 32 while their
     // workgroups are in flight together (four to a CU): min-p 0.05 over 240
-    // rows of 8000: 62 us with 32, 51 with 4 (one workgroup a row: 52)
+    // rows of 8000: 62 us with 32, 30 with 4 (one workgroup a row: 51)
     a.lnp = LNP_MAX;
     while (a.lnp > 0 && ((int64_t)rows << a.lnp) > 4LL * ctx->cu_count && a.V <= (PART_MAX << (a.lnp - 1))) a.lnp--;
     if (a.pen_on || a.sel) {
