@@ -45,7 +45,7 @@ constexpr uint32_t FTOP = 1u << 24;    // fold: ulps from 0 to the top of a bina
 constexpr uint32_t FSAT = 1u << 26;    // fold: saturation of a composed step
 constexpr int FOLD_SEQ = 1024;         // folds: leading elements added by one thread
 constexpr int LBAND = 14, BAND = 1 << LBAND;   // sorted band held in LDS as u64 keys
-constexpr int HIST_MAX = 4096;         // penalty window input limit (4 per thread)
+constexpr int HIST_MAX = 4096;         // penalty window input limit
 constexpr int VMAX = 262144;           // ids fit the low 18 bits of a key
 // a band in candidate order: a block radix sort of 16 keys per thread, each
 // key (desc_key, id) packed into 50 bits, 5 bits per pass with match ranking
@@ -920,6 +920,7 @@ struct DistArgs {
     float ln_min_p;             // logf(min_p), evaluated by the host's libm
     int pen_on;
     float* pen;                 // [rows][V] penalised copies (pen_on)
+    int pen_row;                // made by the row's own workgroup (dist_kernel<0>), not by front_kernel's parts
     int32_t* sid;               // [rows][V] candidate ids in candidate order
     float* sl;                  // [rows][V] their (penalised, untempered) logits
     float* pr;                  // [rows][V] their probabilities
@@ -936,38 +937,44 @@ struct DistArgs {
 // Penalties (lib.rs:233-266): every token of the window carries its penalised
 // logit.  The window is the last penalty_last_n of the history (valid entries,
 // oldest first) followed by the row's preceding drafts (Sampler::accept after
-// each kept draft, engine.rs:2368-2369).  Per row, once: its distinct tokens
-// of the vocabulary with their counts (in e2's space, free until the band
-// parts), which front_kernel's parts apply.
-__global__ __launch_bounds__(FT) void window_kernel(DistArgs a)
+// each kept draft, engine.rs:2368-2369).
+struct Window {
+    const int32_t *hist, *drafts;
+    int hist_len, nd, last_n;
+};
+__device__ __forceinline__ Window row_window(const DistArgs& a, int row)
 {
-    constexpr int HPT = HIST_MAX / FT;
-    __shared__ int win[HIST_MAX + 16];
-    __shared__ Small sm;
-    const int row = blockIdx.x, tid = threadIdx.x;
-    const int32_t *hist = nullptr, *drafts = nullptr;
-    int nd = 0;
+    Window w{nullptr, nullptr, a.hist_len, 0, a.prm.penalty_last_n};
     if (a.direct) {
-        if (a.hist) hist = a.hist + (size_t)row * a.hist_len;
+        if (a.hist) w.hist = a.hist + (size_t)row * a.hist_len;
     } else {
         const int b = row < a.nrow_p ? row / (a.k + 1) : (row - a.nrow_p) / a.k;
-        nd = row < a.nrow_p ? row % (a.k + 1) : (row - a.nrow_p) % a.k;
-        if (a.hist) hist = a.hist + (size_t)b * a.hist_len;
-        drafts = a.draft + (size_t)b * a.k;
+        w.nd = row < a.nrow_p ? row % (a.k + 1) : (row - a.nrow_p) % a.k;
+        if (a.hist) w.hist = a.hist + (size_t)b * a.hist_len;
+        w.drafts = a.draft + (size_t)b * a.k;
     }
-    if (tid < SWV) sm.scan[tid] = 0;           // (the block scan reads SWV wave sums)
-    if (tid == 0) sm.iv[0] = 0;
+    return w;
+}
+
+// use(token, count) once, in any order, for each distinct token below V of
+// the window; for workgroups of NT threads, win in LDS
+template <int NT, class U>
+__device__ __forceinline__ void window_tokens(const Window& w, int V, int* win, Small* sm, U use)
+{
+    constexpr int HPT = HIST_MAX / NT;
+    const int tid = threadIdx.x;
+    if (tid < SWV) sm->scan[tid] = 0;          // (the block scan reads SWV wave sums)
     int tok[HPT], c = 0;
 #pragma unroll
     for (int q = 0; q < HPT; q++) {
         const int i = tid * HPT + q;
-        tok[q] = hist && i < a.hist_len ? hist[i] : -1;
+        tok[q] = w.hist && i < w.hist_len ? w.hist[i] : -1;
         c += tok[q] >= 0 ? 1 : 0;
     }
     __syncthreads();
     uint32_t L;
-    uint32_t p = block_excl_scan((uint32_t)c, &sm, &L);
-    const int total = (int)L + nd, cap = a.prm.penalty_last_n;
+    uint32_t p = block_excl_scan((uint32_t)c, sm, &L);
+    const int total = (int)L + w.nd, cap = w.last_n;
     const int start = total > cap ? total - cap : 0;
     const int wn = total - start;
 #pragma unroll
@@ -977,16 +984,14 @@ __global__ __launch_bounds__(FT) void window_kernel(DistArgs a)
             p++;
         }
     }
-    for (int d = tid; d < nd; d += FT) {
+    for (int d = tid; d < w.nd; d += NT) {
         const int at = (int)L + d;
-        if (at >= start) win[at - start] = drafts[d];
+        if (at >= start) win[at - start] = w.drafts[d];
     }
     __syncthreads();
-    int2* out = (int2*)(a.e2 + (size_t)row * BAND);
-    static_assert(BAND / 2 >= HIST_MAX + 16, "the window's tokens fit");
-    for (int i = tid; i < wn; i += FT) {
+    for (int i = tid; i < wn; i += NT) {
         const int t = win[i];
-        if (t < 0 || t >= a.V) continue;
+        if (t < 0 || t >= V) continue;
         bool first = true;
         int count = 0;
 #pragma unroll 8
@@ -996,10 +1001,41 @@ __global__ __launch_bounds__(FT) void window_kernel(DistArgs a)
                 count++;
             }
         }
-        if (first) out[atomicAdd(&sm.iv[0], 1)] = int2{t, count};   // (applied in any order)
+        if (first) use(t, count);
     }
+}
+
+__device__ __forceinline__ float penalised(float l, int count, float repeat, float freq, float present)
+{
+    if (l <= 0.0f) l *= repeat;
+    else l /= repeat;
+    const float sub = (float)count * freq;
+    return l - (sub + present);
+}
+
+// a row's penalised copy by its one workgroup (not inlined: its registers
+// would be spilled across dist_kernel<0>, 300 us without filters for 270)
+__device__ __noinline__ void penalise_row(const float* lg, float* pen, int V, Window w, float repeat, float freq,
+                                          float present, int* win, Small* sm)
+{
+    strided(V, [&](int i) { return lg[i]; }, [&](int i, float l) { pen[i] = l; });
+    window_tokens<SB>(w, V, win, sm, [&](int t, int count) { pen[t] = penalised(lg[t], count, repeat, freq, present); });
     __syncthreads();
-    if (tid == 0) a.st[row].wn = sm.iv[0];
+}
+
+// For the parts of front_kernel: the window's tokens and counts per row, once
+// (in e2's space, free until the band parts)
+__global__ __launch_bounds__(FT) void window_kernel(DistArgs a)
+{
+    __shared__ int win[HIST_MAX + 16];
+    __shared__ Small sm;
+    const int row = blockIdx.x;
+    if (threadIdx.x == 0) sm.iv[0] = 0;
+    int2* out = (int2*)(a.e2 + (size_t)row * BAND);
+    static_assert(BAND / 2 >= HIST_MAX + 16, "the window's tokens fit");
+    window_tokens<FT>(row_window(a, row), a.V, win, &sm, [&](int t, int count) { out[atomicAdd(&sm.iv[0], 1)] = int2{t, count}; });
+    __syncthreads();
+    if (threadIdx.x == 0) a.st[row].wn = sm.iv[0];
 }
 
 // row `row` of the logits as given, and (the penalised copy when penalties
@@ -1179,12 +1215,7 @@ __global__ __launch_bounds__(FT) void front_kernel(DistArgs a)
         for (int i = tid; i < wn; i += FT) {
             const int2 t = w[i];
             if (t.x < i0 || t.x >= i1) continue;
-            float l = x[t.x - i0];
-            if (l <= 0.0f) l *= a.prm.penalty_repeat;
-            else l /= a.prm.penalty_repeat;
-            const float sub = (float)t.y * a.prm.penalty_freq;
-            l -= sub + a.prm.penalty_present;
-            x[t.x - i0] = l;
+            x[t.x - i0] = penalised(x[t.x - i0], t.y, a.prm.penalty_repeat, a.prm.penalty_freq, a.prm.penalty_present);
         }
         __syncthreads();
         float* pen = a.pen + (size_t)row * V + i0;
@@ -1422,6 +1453,9 @@ __global__ __launch_bounds__(SB) void dist_kernel(DistArgs a)
     float* sl = a.sl + off;
     float* pr = a.pr + off;
     const float* lg = row_logits(a, row);
+    if (PH == 0 && a.pen_row)
+        penalise_row(row_given(a, row), a.pen + off, V, row_window(a, row), P.penalty_repeat, P.penalty_freq,
+                     P.penalty_present, (int*)keys, sm);
 
     if (PH == 0 && P.temp <= 0.0f) {                                  // :324-337 point mass at the first maximum
         const int best = block_argmax([&](int i) { return lg[i]; }, V, 0, sm);
@@ -2010,15 +2044,16 @@ cpv_status dist_launch(cpv_ctx* ctx, DistArgs& a, int rows)
     const size_t lds = SAMPLE_LDS_KEYS + sizeof(Small) + sizeof(FoldLds);
     if (lds > ctx->lds_max) return cpv_fail(ctx, CPV_EUNSUPPORTED, "sampler: needs %zu bytes of LDS", lds);
     const int e0 = cpv_prof_mark(ctx);
-    // Penalties: the penalised rows first (front_kernel).  Top-p: the maximum
-    // and the exponentials over EXP_SPLIT workgroups per row; then, when two
-    // workgroups per row fit the CUs, the index-order sum and the first band
-    // side by side (two workgroups per row), then the rest.  (Penalised rows
-    // past that: 240 rows 720 us with the exponentials ahead, 617 without.)
+    // Top-p: the maximum and the exponentials over EXP_SPLIT workgroups per
+    // row; then, when two workgroups per row fit the CUs, the index-order sum
+    // and the first band side by side (two workgroups per row), then the rest.
+    // (Penalised rows past that: 240 rows 720 us with the exponentials ahead,
+    // 617 without; and short ones, by their own workgroup: V 4000 88 to 181 us
+    // split, 75 to 97 not; V 8000 126 to 176 against 136 to 154.)
     const cpv_sampler_params& P = a.prm;
     const bool top_k = P.top_k > 0 && P.top_k < a.V;
     a.pre_exp = P.temp > 0.0f && !top_k && !(P.min_p > 0.0f) && P.top_p < 1.0f && rows <= 65535 &&
-                (!a.pen_on || 2 * rows <= ctx->cu_count);
+                (!a.pen_on || (2 * rows <= ctx->cu_count && a.V >= 6144));
     // Top-k and min-p: the candidates selected by parts of the row first, at
     // every row count (V 151936, k = 4, us a call against one workgroup a
     // row: top-k 40 at 9 rows 112 -> 52, at 240 rows 182 -> 156; min-p 129 ->
@@ -2031,7 +2066,14 @@ cpv_status dist_launch(cpv_ctx* ctx, DistArgs& a, int rows)
     // rows of 8000: 62 us with 32, 30 with 4 (one workgroup a row: 51)
     a.lnp = LNP_MAX;
     while (a.lnp > 0 && ((int64_t)rows << a.lnp) > 4LL * ctx->cu_count && a.V <= (PART_MAX << (a.lnp - 1))) a.lnp--;
-    if (a.pen_on || a.sel) {
+    // Penalties: the penalised rows first, by parts (front_kernel), or, where
+    // nothing else comes of the parts, in the row's own workgroup at V up to
+    // 65536 or from 49 rows on (temperature 0: V 32000 17 -> 15 us at 1 row, 30
+    // -> 24 at 240; V 64000 19.7, 20.3 at 1; V 151936 27 -> 34 at 1, 37.7 ->
+    // 38.4 at 40, 45 -> 40 at 72, 100 -> 74 at 240; top-k 300 86 -> 94, 97 ->
+    // 100, 107 -> 103, 168 -> 141)
+    a.pen_row = a.pen_on && !a.sel && !a.pre_exp && (a.V <= 65536 || rows > 48);
+    if ((a.pen_on && !a.pen_row) || a.sel) {
         if (a.pen_on) window_kernel<<<(unsigned)rows, FT, 0, ctx->stream>>>(a);
         const size_t part_b = a.pen_on ? (size_t)(((a.V + (1 << a.lnp) - 1) >> a.lnp) + 3 & ~3) * 4 : 0;
         front_kernel<<<dim3((unsigned)rows, 1u << a.lnp), FT, part_b, ctx->stream>>>(a);
