@@ -1470,27 +1470,21 @@ __global__ __launch_bounds__(SB) void dist_kernel(DistArgs a)
 
     constexpr bool split = PH == 1 || PH == 2;
     const bool top_k = !split && P.top_k > 0 && P.top_k < V;         // :272-280
-    const bool min_p = !split && !top_k && P.min_p > 0.0f;           // :281-295
-    const bool top_p = PH == 3 ? false : split || (!top_k && !min_p && P.top_p < 1.0f); // :296-316
+    const bool min_p = PH == 3 && !top_k;                            // :281-295 (always by parts)
+    const bool top_p = PH == 3 ? false : split || (!top_k && P.top_p < 1.0f); // :296-316
     // (the split build needs no maximum here: exp_kernel has used it, and
     // top-p's final softmax is relative to the first candidate)
     float mx = 0.0f;
-    if (PH == 3 && a.sel < 0) {
-        mx = parts_max(a.st[row]);
-    } else if (PH == 0 && !a.pre_exp && !top_k) {
-        mx = block_max([&](int i) { return lg[i]; }, V, sm);
-    }
+    if (PH == 0 && !a.pre_exp && !top_k) mx = block_max([&](int i) { return lg[i]; }, V, sm);
     int n;
-    if (PH != 0 || top_k || min_p || top_p) {
+    if (PH != 0 || top_k || top_p) {
         int M = 0, emitted = 0;
         unsigned long long last = 0;
         if (top_k) {
             M = P.top_k > P.min_keep ? P.top_k : P.min_keep;
             if (M > V) M = V;
         } else if (min_p) {
-            const float floor_l = mx + a.ln_min_p;
-            if (PH == 3 && a.sel < 0) M = cpv_wave_reduce((tid & 63) < EXP_SPLIT ? a.st[row].fval[tid & 63] : 0, cpv_op_add());
-            else M = block_count([&](int i) { return lg[i] >= floor_l; }, V, sm);
+            M = cpv_wave_reduce((tid & 63) < EXP_SPLIT ? a.st[row].fval[tid & 63] : 0, cpv_op_add());
         } else {
             // softmax over the vocabulary in index order, then the probe:
             // the smallest of 1024, 8192, ... (capped at V) whose sorted
@@ -1664,7 +1658,7 @@ __global__ __launch_bounds__(SB) void dist_kernel(DistArgs a)
     }
     // :371-374 temperature, then softmax over the survivors (:461-471)
     const float T = P.temp;
-    const float mx2 = (PH != 0 || top_k || min_p || top_p ? sl[0] : mx) / T;
+    const float mx2 = (PH != 0 || top_k || top_p ? sl[0] : mx) / T;
     __syncthreads();
     if (top_p && PH == 2 && a.st[row].np > 0 && n <= a.st[row].cnt) {
         // the survivors lie in the first band: its parts' e2 and composed
@@ -2060,7 +2054,7 @@ cpv_status dist_launch(cpv_ctx* ctx, DistArgs& a, int rows)
     // 54 and 215 -> 138); top-k up to FRONT_K, as a part may keep FCAP keys
     // and whole bins come with them (300: the bands, 107 us at 9 rows)
     const int kk = P.top_k > P.min_keep ? P.top_k : P.min_keep;
-    a.sel = P.temp > 0.0f ? top_k ? (kk <= FRONT_K ? kk : 0) : P.min_p > 0.0f ? -1 : 0 : 0;
+    a.sel = !(P.temp <= 0.0f) ? top_k ? (kk <= FRONT_K ? kk : 0) : P.min_p > 0.0f ? -1 : 0 : 0;
     // Parts: a power of two of at most PART_MAX elements each, 32 while their
     // workgroups are in flight together (four to a CU): min-p 0.05 over 240
     // rows of 8000: 62 us with 32, 30 with 4 (one workgroup a row: 51)
