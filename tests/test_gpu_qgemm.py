@@ -9,6 +9,8 @@ the weights (12 and 24 rows check the partial and split launches; Q4_K above
 (Q6_K, Q8_0) every type runs on its wide (prefill) kernel, held to the same
 bar.
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -114,8 +116,9 @@ def test_qgemm_wide_bit_exact_small(ctx, tname, n, k, m):
 @pytest.mark.parametrize("tname", ["q4_k", "q6_k", "q8_0"])
 @pytest.mark.parametrize("m", [9, 16, 17, 33, 49, 65, 81, 97, 113, 128, 129, 145, 255])
 def test_qgemm_wide_row_blocks(ctx, tname, m):
-    # every number of 16-row blocks a workgroup holds, with one row in the last
-    # block or all; weight rows past a tile; 11 units, which no slice count divides
+    # few tiles: 1 to 3 16-row blocks a workgroup, K in slices (11 units, which
+    # no slice count divides), with one row in the last block or all; weight
+    # rows past a tile
     y, ref = run_case(ctx, TYPES[tname], 131, 2816, m)
     assert np.array_equal(y.view(np.uint32), ref.view(np.uint32)), np.abs(y - ref).max()
 
@@ -138,15 +141,55 @@ def test_qgemm_units_below_the_scale_range(ctx, m):
     assert np.array_equal(y, cpvo.qgemm(t, wq, z))
 
 
-@pytest.mark.parametrize("tname", ["q4_k", "q6_k", "q8_0"])
-def test_qgemm_wide_whole_and_sliced(ctx, tname):
-    # more (tile, row block) pairs than workgroups in flight: whole rounds run
-    # over all of K, the rest in K slices through the accumulator; twice, as
-    # the accumulator has to be zero again
-    t, n, k, m = TYPES[tname], 64 * 810 + 3, 2048, 40
-    for seed in (0, 1):
-        y, ref = run_case(ctx, t, n, k, m, seed=seed)
-        assert np.array_equal(y.view(np.uint32), ref.view(np.uint32)), np.abs(y - ref).max()
+def raw_blocks(t, n, k, seed=0):
+    """ggml blocks of n rows [n][bytes]: random codes and sub-block scales, a
+    tenth of the block scales 30 times the others."""
+    rng = np.random.default_rng(seed)
+    size, elems, at = {cpvo.Q8_0: (34, 32, (0,)), cpvo.Q4_K: (144, 256, (0, 2)), cpvo.Q6_K: (210, 256, (208,))}[t]
+    raw = rng.integers(0, 256, size=(n * (k // elems), size), dtype=np.uint8)
+    for o in at:
+        d = rng.uniform(0.5, 1.5, raw.shape[0]) * np.where(rng.random(raw.shape[0]) < 0.1, 3e-2, 1e-3)
+        raw[:, o:o + 2] = d.astype(np.float16).view(np.uint8).reshape(-1, 2)
+    return raw.reshape(n, -1)
+
+
+def wide_plan(ctx, t, n, k, m):
+    """cpv_qgemm_wide_plan: 16-row blocks per workgroup, row blocks, pairs over
+    all of K, K slices of the other pairs, units a slice."""
+    ctx.lib.cpv_qgemm_wide_plan.argtypes = [ctypes.c_int] + [ctypes.c_int64] * 3 + [ctypes.c_int, ctypes.c_int * 5]
+    out = (ctypes.c_int * 5)()
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert ctx.lib.cpv_qgemm_wide_plan(t, n, k, m, cus, out)
+    return list(out)
+
+
+@pytest.mark.parametrize("tname,nmt", [(t, b) for t, lo, hi in (("q4_k", 2, 8), ("q6_k", 1, 8), ("q8_0", 1, 4))
+                                       for b in range(lo, hi + 1)])
+def test_qgemm_wide_whole_and_sliced(ctx, tname, nmt):
+    # every number of 16-row blocks a workgroup may hold: whole rounds of
+    # workgroups over all of K (9 units, in both staging buffers) and one pair
+    # past them in two K slices through the accumulator, which has to be zero
+    # again for the next row count; one row in the last block, then all.  Every
+    # output against the skinny kernels', some tiles' against the oracle's.
+    t = TYPES[tname]
+    tiles = 1536 if (tname, nmt) == ("q8_0", 4) else 768 if tname == "q8_0" or nmt <= 2 else 512
+    n, k = 64 * tiles + 3, 2304
+    wq = raw_blocks(t, n, k)
+    rows = np.r_[0:64, n // 2:n // 2 + 64, n - 130:n]
+    w = ctx.upload_weight(t, wq, n, k)
+    for m in (max(9, 16 * nmt - 15), 16 * nmt):
+        assert wide_plan(ctx, t, n, k, m) == [nmt, 1, tiles, 2, 5]
+        print(f"case type={tname} n={n} k={k} m={m}", flush=True)
+        x = np.random.default_rng(m).normal(0, 1, size=(m, k)).astype(np.float32)
+        x[m // 2] *= 1e-3
+        xt = torch.from_numpy(x).cuda()
+        y = ctx.qgemm(w, xt)
+        for r in range(0, m, 8):
+            ys = ctx.qgemm(w, xt[r:r + 8].contiguous())
+            assert torch.equal(y[r:r + 8].view(torch.int32), ys.view(torch.int32)), r
+        ref = cpvo.qgemm(t, wq[rows], x)
+        assert np.array_equal(y.cpu().numpy()[:, rows].view(np.uint32), ref.view(np.uint32))
+    w.free()
 
 
 def test_qgemm_wide_many_weight_rows():
