@@ -8,6 +8,8 @@ chunks in chunk order.  So the device result does not depend on its grid or
 on the number of query rows per call.  The contract itself is held within
 2^-12 max|v| + 2^-15 of binary64 attention by the oracle's own tests.
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -74,6 +76,45 @@ def test_many_rows_take_limb_caches(ctx, t, h, hkv, d, n_past):
     # 16-row segments), 515 query rows, a last block of 3; 1028 over 17
     # chunks, in blocks of 48
     close(*run(ctx, t, h, hkv, d, n_past, None, extra_rows=3))
+
+
+@pytest.mark.parametrize("big", [False, True])
+@pytest.mark.parametrize("h,hkv,d,n_past,t,blocks", [(40, 8, 128, 3600, 320, [309, 11]), (32, 4, 64, 3200, 800, [733, 67])])
+def test_many_rows_in_two_token_blocks(h, hkv, d, n_past, t, blocks, big):
+    # the limb caches of one conversion at the front of a workspace that grows
+    # within the call, under two token blocks (the first sees fewer rows than
+    # were converted), with a V stride far above the rows; with values of
+    # magnitude 512 and up (the top value limb) and without.  Against calls of
+    # fewer than 512 query rows per KV head, which take the f16 caches, and the
+    # oracle on both sides of the block boundary and at the end.
+    from codpiece_amd.runtime import Context
+    ctx = Context(0)                               # (no workspace yet)
+    ctx.lib.cpv_attn_takes_limbs.argtypes = [ctypes.c_int64] + [ctypes.c_int] * 4
+    chunks = (n_past + t + 127) // 128
+    tb = 192 * 2**20 // (h * chunks * (4 * d + 12) + 1)
+    step = 511 // (h // hkv)
+    assert [tb, t - tb] == blocks and ctx.lib.cpv_attn_takes_limbs(n_past, t, h, hkv, d)
+    assert not ctx.lib.cpv_attn_takes_limbs(n_past + t - step, step, h, hkv, d)
+    rng = np.random.default_rng(n_past + big)
+    n = n_past + t
+    k, v, _ = make(rng, n, hkv, d)
+    if big:
+        mask = (rng.random(n) < 0.05)[:, None] & (rng.random(hkv * d) < 0.3)[None, :]
+        v = np.where(mask, cpvo.f32_to_f16_bits((rng.normal(size=v.shape) * 3000).astype(np.float32)), v)
+    vt = np.full((hkv * d, 8192), 0x7e00, dtype=np.uint16)    # (NaN past the rows: never read into a result)
+    vt[:, :n] = v.T
+    q = rng.normal(size=(t, h, d)).astype(np.float32)
+    scale = np.float32(1) / np.sqrt(np.float32(d))
+    qt, kt, vtt = torch.from_numpy(q).cuda(), torch.from_numpy(k.view(np.int16)).cuda(), torch.from_numpy(vt.view(np.int16)).cuda()
+    print(f"case h={h} hkv={hkv} d={d} n_past={n_past} t={t} big={big}", flush=True)
+    got = ctx.attn(qt, kt, vtt, n_past, None, hkv, float(scale))
+    for t0 in range(0, t, step):
+        part = ctx.attn(qt[t0:t0 + step].contiguous(), kt, vtt, n_past + t0, None, hkv, float(scale))
+        assert torch.equal(got[t0:t0 + step], part), t0
+    got = got.cpu().numpy()
+    for t0 in (0, tb - 1, t - 2):
+        close(got[t0:t0 + 2], cpvo.attn(q[t0:t0 + 2], k[:n_past + t0 + 2], v[:n_past + t0 + 2], n_past + t0, None, scale))
+    ctx.close()
 
 
 @pytest.mark.parametrize("n_ctx", [8192, 32768])
