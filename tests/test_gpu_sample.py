@@ -122,6 +122,29 @@ def test_distribution_selected_by_fewer_parts(ctx, rows, v):
         check_dist(ctx, x, cpvo.SamplerParams(**c), hist if "penalty_repeat" in c else None)
 
 
+@pytest.mark.parametrize("v", [400, 4000, 151936])
+def test_candidate_order_of_nan_and_infinities(ctx, v):
+    # the candidate order of logits that no comparison orders: a NaN before
+    # every number (one of the other sign after them), by parts and by bands
+    rng = np.random.default_rng(v)
+    x = spiked(rng, (4, v))
+    x[0, rng.integers(0, v, 3)] = np.nan
+    x[1, rng.integers(0, v, 3)] = np.uint32(0xffc00000).view(np.float32)
+    x[2, rng.integers(0, v, 5)] = np.inf
+    x[3] = -np.inf
+    x[3, ::max(1, v // 20)] = 1.0
+    b = np.where(x == 0, np.float32(0), x).view(np.uint32)
+    key = ~np.where(b >> 31, ~b, b | np.uint32(1 << 31))
+    order = np.argsort(key, axis=1, kind="stable")
+    top = np.fmax.reduce(x, axis=1)
+    for c in (dict(top_k=20), dict(top_k=300), dict(min_p=0.05)):
+        ids, _, n = ctx.distribution(torch.from_numpy(x).cuda(), dev_params(cpvo.SamplerParams(temp=0.8, **c)))
+        ids, n = ids.cpu().numpy(), n.cpu().numpy()
+        for r in range(4):
+            want = c["top_k"] if "top_k" in c else np.count_nonzero(x[r] >= top[r] + np.float32(np.log(np.float32(0.05))))
+            assert n[r] == want and np.array_equal(ids[r, :want], order[r, :want]), (c, r, n[r], want)
+
+
 @pytest.mark.parametrize("rows", [60, 140])
 def test_distribution_top_p_row_counts(ctx, rows):
     # top-p builds: the maximum and exponentials over many workgroups per
