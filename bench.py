@@ -395,7 +395,9 @@ def gemm_bench(torch, ctx, seed, rotate_bytes=512e6):
     type) x f32 activations ~N(0, 1) of M rows, for each of
     GEMM_SHAPES and M in {1, 5, 8, 16}, and at 256 rows (a prefill chunk's:
     `TOP_s` is its int8 rate); `kernel` "wide" marks the launches the library
-    gave its wide kernels (Q6_K and Q8_0 from 9 rows, Q4_K from 17).  Each shape's weights are uploaded in
+    gave its wide kernels (Q6_K and Q8_0 from 9 rows, Q4_K from 17), whose
+    recorded launch writes the outputs too (with the sliced pairs' second
+    kernel; the skinny ones' finalize is in `us_call` only).  Each shape's weights are uploaded in
     enough copies to cover `rotate_bytes` (more than the 256 MB last-level
     cache), and consecutive calls rotate through them, so every call streams
     its weights from HBM.  `us` is the GEMM kernels' time per call (the

@@ -22,8 +22,9 @@
 // Kernels: chunk (grid: chunk x KV head x query block of 32, 48 or 80 rows;
 // scores on the MFMA, then the chunk's softmax and its P_c in the same
 // workgroup) and fold (one block per query row), and over the API's caches a
-// first launch that makes the query rows' limbs once.  Scratch in the context
-// workspace: P (per chunk and query row, D f32: [chunks][T*H][D] for a
+// first launch that makes the query rows' limbs once, or, for a prompt chunk
+// of many rows, one that makes the caches into limb caches (limbs_pay).
+// Scratch in the context workspace: those limb caches, P (per chunk and query row, D f32: [chunks][T*H][D] for a
 // consumer's fold, [T*H][chunks][D] for the fold here), m [chunks][T*H] f32,
 // Z [chunks][T*H] int64, the query limbs.
 //
@@ -33,7 +34,8 @@
 // (a chunk's 128 exponents of one head in 512 contiguous bytes), V as vq's
 // limbs, [h_kv * d][v_stride / 16][4][16].  The API's caches (cpv_attn) are f16:
 // K [n_ctx][h_kv * d] and the transposed V [h_kv * d][v_stride] (the
-// reference's non-FA V layout, qwen35.rs:580-586), converted in the kernel.
+// reference's non-FA V layout, qwen35.rs:580-586), converted in the chunk
+// kernel or, once for all its query blocks, by kv_limbs_kernel.
 // Either way the KV axis is the reduction axis of P V.
 #include <math.h>
 
@@ -793,8 +795,9 @@ cpv_status attn_block(cpv_ctx* ctx, const float* q, const uint16_t* kc, const ui
     // once for all of them, not once per 48-row block.
     // A prompt chunk's many rows over limb caches take 48-row blocks from 16
     // chunks on too, at d = 128 (40/8 heads, 512 tokens after 3584: 429 -> 411
-    // us, 24/4: 268 -> 258; after 1000, 9 to 12 chunks, no gain; at d = 64
-    // 32/4: 222 -> 233).
+    // us; 32-row / 48-row time over 40/8, 32/8, 24/4 and 28/4 heads, 1600 to
+    // 7000 rows before and 1024 to 2560 query rows: 0.925 to 1.014, one 1.024;
+    // after 1000, 9 to 12 chunks, no gain; at d = 64 32/4: 222 -> 233).
     const bool many = D == 128 && vl && LR >= 1024 && nchunk >= 16;
     const bool wide = many || (LR > QB_CHAIN && (int64_t)nchunk * Hkv >= WIDE_UNITS);
     const bool tree_blk = wide && !vl && LR > QB_WIDE && LR <= QB_TREE;

@@ -17,8 +17,9 @@
 // activation codes of one unit are staged in LDS for the four waves,
 // double-buffered, while the next unit's codes and weights are in flight.  In
 // the MFMA's lane layout (A row and B column = lane % 16, C rows 4 (lane / 16)
-// + i of column lane % 16) each lane holds one weight row, so its scales are
-// decoded once per unit.
+// + i of column lane % 16) a lane of the K-quants' kernel holds one weight row,
+// so its scales are decoded once per unit; one of Q8_0's (the weights as A)
+// holds one activation row and four weight rows.
 #include <math.h>
 
 #include "cpv_internal.h"
@@ -668,8 +669,10 @@ namespace {
 // Rows per workgroup and the deal of the (tile, row block) pairs over the
 // chip's slots (workgroups in flight).  Whole rounds of pairs run over all of
 // K; the pairs that are left run in ks K slices of at least 4 units each.
-// Chosen by an estimate in us, from 5120, 7168, 12288, 17408 and 34816 x 5120
-// and 5120 x 17408 at 64 to 256 rows: a unit of nmt row blocks takes 0.5 +
+// Chosen by an estimate in us, fitted to 5120, 7168, 12288, 17408 and 34816 x
+// 5120 and 5120 x 17408 at 64 to 256 rows (at 9 to 48, those and five smaller
+// weights, whole calls: Q8_0 0.60 to 0.92 of the fixed 64-row blocks' and their
+// finalize launch's time, the K-quants' none above theirs): a unit of nmt row blocks takes 0.5 +
 // 0.315 nmt with two workgroups on a CU (Q8_0: 0.95 nmt with three) and 0.62
 // of that with one, a workgroup's start (row exponents, first loads) 3, and a
 // million atomic adds of a slice's sums 3.5 (they bypass the XCD's L2).  E.g.

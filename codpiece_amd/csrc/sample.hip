@@ -2051,7 +2051,7 @@ cpv_status dist_launch(cpv_ctx* ctx, DistArgs& a, int rows)
     // Top-k and min-p: the candidates selected by parts of the row first, at
     // every row count (V 151936, k = 4, us a call against one workgroup a
     // row: top-k 40 at 9 rows 112 -> 52, at 240 rows 182 -> 156; min-p 129 ->
-    // 54 and 215 -> 138); top-k up to FRONT_K, as a part may keep FCAP keys
+    // 54 and 215 -> 138); top-k up to FRONT_K, as a part may keep 512 keys
     // and whole bins come with them (300: the bands, 107 us at 9 rows)
     const int kk = P.top_k > P.min_keep ? P.top_k : P.min_keep;
     a.sel = !(P.temp <= 0.0f) ? top_k ? (kk <= FRONT_K ? kk : 0) : P.min_p > 0.0f ? -1 : 0 : 0;
@@ -2062,14 +2062,14 @@ cpv_status dist_launch(cpv_ctx* ctx, DistArgs& a, int rows)
     while (a.lnp > 0 && ((int64_t)rows << a.lnp) > 4LL * ctx->cu_count && a.V <= (PART_MAX << (a.lnp - 1))) a.lnp--;
     // Penalties: the penalised rows first, by parts (front_kernel), or, where
     // nothing else comes of the parts, in the row's own workgroup at V up to
-    // 65536 or from 49 rows on (temperature 0: V 32000 17 -> 15 us at 1 row, 30
-    // -> 24 at 240; V 64000 19.7, 20.3 at 1; V 151936 27 -> 34 at 1, 37.7 ->
+    // 65536 or from 49 rows on (by parts -> by the row's workgroup, us a call:
+    // temperature 0 at V 32000 17 -> 15 at 1 row, 30 -> 24 at 240; V 64000 19.7 -> 20.3 at 1; V 151936 27 -> 34 at 1, 37.7 ->
     // 38.4 at 40, 45 -> 40 at 72, 100 -> 74 at 240; top-k 300 86 -> 94, 97 ->
     // 100, 107 -> 103, 168 -> 141)
     a.pen_row = a.pen_on && !a.sel && !a.pre_exp && (a.V <= 65536 || rows > 48);
     if ((a.pen_on && !a.pen_row) || a.sel) {
         if (a.pen_on) window_kernel<<<(unsigned)rows, FT, 0, ctx->stream>>>(a);
-        const size_t part_b = a.pen_on ? (size_t)(((a.V + (1 << a.lnp) - 1) >> a.lnp) + 3 & ~3) * 4 : 0;
+        const size_t part_b = a.pen_on ? (size_t)((((a.V + (1 << a.lnp) - 1) >> a.lnp) + 3) & ~3) * 4 : 0;
         front_kernel<<<dim3((unsigned)rows, 1u << a.lnp), FT, part_b, ctx->stream>>>(a);
     }
     if (!a.pen_on && !a.sel && a.pre_exp) rowmax_part_kernel<<<dim3(EXP_SPLIT, (unsigned)rows), 256, 0, ctx->stream>>>(a);

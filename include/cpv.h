@@ -86,8 +86,8 @@ cpv_status  cpv_get_rows(cpv_ctx* ctx, const cpv_weight* w, const int32_t* rows_
  * result does not depend on how the K loop is split.
  * Replaces every ggml_mul_mat on the verify path (qwen35.rs:2779-2782,2797,
  * 3029,3047,3051,3197; mtp_graph.rs:184,209-212,230).  x_dev: f32 [m][k];
- * y_dev: f32 [m][n_rows]; 1 <= m <= 256 (Q4_K from 32 rows on: the wide
- * prefill kernel, the same sums). */
+ * y_dev: f32 [m][n_rows]; 1 <= m <= 256 (Q4_K from 17 rows and Q6_K
+ * and Q8_0 from 9 on: the wide prefill kernels, the same sums). */
 cpv_status  cpv_qgemm(cpv_ctx* ctx, const cpv_weight* w, const float* x_dev, int64_t m,
                       float* y_dev);
 
