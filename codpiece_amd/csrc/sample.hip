@@ -1321,8 +1321,9 @@ __global__ __launch_bounds__(FT) void floor_kernel(DistArgs a)
 // or 0 when a part selected more than it may keep or the M largest cannot be
 // told from more than a key per thread (the caller then emits bands).  A min-p
 // build of more than 3/4 of a key per thread gets all its keys in the key buffer,
-// unsorted: minus their number (emit_band takes them from there; V 32000, B =
-// 1, 2700 keys: 82 us through the bands, 54 so; without the parts 73).  The
+// unsorted: minus their number (emit_band takes them from there; one row of V
+// 32000, N(0, 3), min-p 0.001: 82 us through the bands, 54 so; without the
+// parts 73).  The
 // keys with the M largest logits lie in the first bins of a histogram over
 // the selected keys' own range of desc_key (4096 bins).
 template <bool MOST>   // EXP_SPLIT parts (a fixed layout of the keys: 0.3 us)
